@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/lcodepy_amd.h"
+#include "common.h"
 #include "kernels.h"
 
 using namespace lc3d;
@@ -44,7 +45,6 @@ struct lc3d_ctx {
     double *rowsum = nullptr;
     double *diag = nullptr;   // energy-flux partial sums, 2 DIAG_BLOCKS
     unsigned long long *beam_acc = nullptr;   // beam deposit fixed-point sums, 6 N*N, zero
-    float *fields32 = nullptr;   // FP32-bulk: float32 copies of six float64 fields
     void *tw = nullptr;                                      // FFT twiddles
     uint64_t rf_stages = 0;                                  // RFFT radix plan (packed)
     int rf_cap = 0, rf_tpb = 0, rf_wave = 0;                 // RFFT launch shape
@@ -368,32 +368,26 @@ const int *push_order(const lc3d_ctx *c, const lc3d_sort *s)
                : nullptr;
 }
 
-// as_f32: an FP32-bulk context pushes float64 fields rounded to float32 (the
-// step's first push, from the previous step's full fields).
 int push_sort(lc3d_ctx *c, const lc3d_sort *s, const void *const *f, bool f32, bool first,
-              bool bin, hipStream_t st, bool as_f32 = false)
+              bool bin, bool momenta, hipStream_t st)
 {
     const lc3d_fields6 fl{f[0], f[1], f[2], f[3], f[4], f[5]};
     hipError_t e;
     if (fp32(c)) {
-        if (!f32 && as_f32)
-            e = launch_push_f64_fields_as_f32(push_geom(c, s->n), f6<double>(&fl), c->fields32,
-                                              sort_arrays<float>(s), first, bin,
-                                              bin_state(c, s->column), push_order(c, s), st,
-                                              timer_of(c));
-        else if (f32)
+        if (f32)
             e = launch_push<float, float>(push_geom(c, s->n), f6<float>(&fl), sort_arrays<float>(s),
-                                          first, bin, bin_state(c, s->column), push_order(c, s), st,
+                                          first, bin, momenta, bin_state(c, s->column),
+                                          push_order(c, s), st,
                                           timer_of(c));
         else
             e = launch_push<float, double>(push_geom(c, s->n), f6<double>(&fl),
-                                           sort_arrays<float>(s), first, bin, bin_state(c, s->column),
-                                           push_order(c, s), st, timer_of(c));
+                                           sort_arrays<float>(s), first, bin, momenta,
+                                           bin_state(c, s->column), push_order(c, s), st, timer_of(c));
     } else {
         if (f32) return fail(c, LC3D_EINVAL, "float32 fields need an FP32-bulk context");
         e = launch_push<double, double>(push_geom(c, s->n), f6<double>(&fl),
-                                        sort_arrays<double>(s), first, bin, bin_state(c, s->column),
-                                        push_order(c, s), st, timer_of(c));
+                                        sort_arrays<double>(s), first, bin, momenta,
+                                        bin_state(c, s->column), push_order(c, s), st, timer_of(c));
     }
     if (e != hipSuccess) return hip_fail(c, e, "push");
     return LC3D_OK;
@@ -507,14 +501,15 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
     c->prm.declustering_taps = nullptr;
     (void)hipGetDevice(&c->device);
     const size_t nn = (size_t)N * N;
-    const size_t nblocks = (size_t)scan_tiles((int64_t)nn);
+    const size_t nkeys = (size_t)cell_keys(N);   // cells in list order
+    const size_t nblocks = (size_t)scan_tiles((int64_t)nkeys);
     c->nbase = (int)nblocks;
     const bool f32 = p->precision == LC3D_FP32_BULK;
     const size_t tg = f32 ? sizeof(float) : sizeof(double);
     const size_t cap = (size_t)std::max<int64_t>(1, c->cap);
-    bool ok = hipMalloc(&c->count, (nn + 1) * sizeof(int)) == hipSuccess &&
-              hipMalloc(&c->start, (nn + 1) * sizeof(int)) == hipSuccess &&
-              hipMalloc(&c->lstart, (nn + 1) * sizeof(int)) == hipSuccess &&
+    bool ok = hipMalloc(&c->count, (nkeys + 1) * sizeof(int)) == hipSuccess &&
+              hipMalloc(&c->start, (nkeys + 1) * sizeof(int)) == hipSuccess &&
+              hipMalloc(&c->lstart, (nkeys + 1) * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->base, nblocks * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->key, cap * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->rank, cap * sizeof(int)) == hipSuccess &&
@@ -525,14 +520,12 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
               hipMalloc(&c->pos, cap * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->big, dense_cell_capacity(cap) * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->nbig, sizeof(int)) == hipSuccess &&
-              hipMalloc(&c->dslot, nn * sizeof(int)) == hipSuccess &&
+              hipMalloc(&c->dslot, nkeys * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->dense, dense_cell_capacity(cap) * 100 * tg) == hipSuccess &&
               hipMalloc(&c->work, 7 * nn * tg) == hipSuccess &&
               hipMalloc(&c->rowsum, N * sizeof(double)) == hipSuccess &&
               hipMalloc(&c->diag, 2 * DIAG_BLOCKS * sizeof(double)) == hipSuccess &&
               hipMalloc(&c->beam_acc, 6 * nn * sizeof(unsigned long long)) == hipSuccess &&
-              (!f32 || hipMalloc(&c->fields32, 6 * fields32_stride(N) * sizeof(float)) ==
-                           hipSuccess) &&
               hipMemset(c->beam_acc, 0, 6 * nn * sizeof(unsigned long long)) == hipSuccess &&
               hipMalloc(&c->lam, N * sizeof(double)) == hipSuccess;
     if (ok && (fft || rfft)) ok = hipMalloc(&c->tw, 2 * (size_t)M * 2 * tg) == hipSuccess;
@@ -600,7 +593,7 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
     if (e == hipSuccess && c->dc_side > 0)
         e = hipMemcpy(c->dc_taps, p->declustering_taps, c->dc_ntaps * sizeof(double),
                       hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemset(c->count, 0, (nn + 1) * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(c->count, 0, (nkeys + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->base, 0, c->nbase * sizeof(int));
     if (e == hipSuccess) e = hipMemset(c->nbig, 0, sizeof(int));
@@ -641,7 +634,6 @@ void lc3d_destroy(lc3d_ctx *c)
     (void)hipFree(c->rowsum);
     (void)hipFree(c->diag);
     (void)hipFree(c->beam_acc);
-    (void)hipFree(c->fields32);
     (void)hipFree(c->tw);
     (void)hipFree(c->tdst);
     (void)hipFree(c->tdct);
@@ -731,7 +723,8 @@ int lc3d_move_smart(lc3d_ctx *c, const lc3d_sort *s, const lc3d_fields6 *f, int3
     if (!c || !sort_ok(c, s) || !f || !f->Ex || !f->Ey || !f->Ez || !f->Bx || !f->By || !f->Bz)
         return fail(c, LC3D_EINVAL, "move_smart: bad arguments");
     const void *fl[6] = {f->Ex, f->Ey, f->Ez, f->Bx, f->By, f->Bz};
-    return push_sort(c, s, fl, field_fp32 != 0, false, false, static_cast<hipStream_t>(stream));
+    return push_sort(c, s, fl, field_fp32 != 0, false, false, true,
+                     static_cast<hipStream_t>(stream));
 }
 
 int lc3d_deposit(lc3d_ctx *c, const lc3d_sort *s, void *ro, void *jx, void *jy, void *jz,
@@ -796,14 +789,14 @@ int lc3d_plasma_step(lc3d_ctx *c, int32_t n_sorts, const lc3d_sort *sorts,
     int r;
     // solver.py:29-42: free stream + push 1 in fields_prev, deposit 1.
     for (int s = 0; s < n_sorts; ++s) {
-        if ((r = push_sort(c, &sorts[s], fprev, false, true, true, st, true))) return r;
+        if ((r = push_sort(c, &sorts[s], fprev, false, true, true, false, st))) return r;
         if ((r = deposit_sort(c, &sorts[s], true, cf, bg_ro, single, st))) return r;
     }
     // solver.py:44-47: solve 1 with fields_prev as predictor; only the half fields are kept.
     if ((r = solve(c, prev, false, prev, rbF, rbP, cp, cf, full, half, false, st))) return r;
     // solver.py:49-57: push 2 in fields_half, deposit 2.
     for (int s = 0; s < n_sorts; ++s) {
-        if ((r = push_sort(c, &sorts[s], fhalf, f32, false, true, st))) return r;
+        if ((r = push_sort(c, &sorts[s], fhalf, f32, false, true, false, st))) return r;
         if ((r = deposit_sort(c, &sorts[s], true, cf, bg_ro, single, st))) return r;
     }
     // solver.py:59-62: solve 2 with fields_half as predictor.
@@ -813,7 +806,7 @@ int lc3d_plasma_step(lc3d_ctx *c, int32_t n_sorts, const lc3d_sort *sorts,
     // deposit instead of by the push), deposit 3.
     for (int s = 0; s < n_sorts; ++s) {
         const bool filter = s == 0 && declust_ok(c, &sorts[s]);
-        if ((r = push_sort(c, &sorts[s], fhalf, f32, false, !filter, st))) return r;
+        if ((r = push_sort(c, &sorts[s], fhalf, f32, false, !filter, true, st))) return r;
         if (filter && (r = noise_filter_sort(c, &sorts[s], st))) return r;
         if ((r = deposit_sort(c, &sorts[s], !filter, cf, bg_ro, single, st))) return r;
     }

@@ -101,6 +101,22 @@ __device__ __forceinline__ int xcd_swizzle(int b, int n) {
     return (b & 7) * (n8 >> 3) + (b >> 3);
 }
 
+// Cell order of the deposit lists and of the particles' visits: strips of
+// STRIP columns (cells along y), walked along x up one strip and down the
+// next, so that any run of consecutive cells is a compact patch of the grid
+// (the push stages the fields around such a patch in LDS).  cell_key is the
+// place of cell (ix, iy) in that order, below cell_keys(N) (the last strip
+// counts STRIP columns whether the grid has them or not).
+constexpr int STRIP = 32;
+__host__ __device__ __forceinline__ int cell_keys(int N) {
+    return (N + STRIP - 1) / STRIP * STRIP * N;
+}
+__device__ __forceinline__ int cell_key(int ix, int iy, int N) {
+    const int strip = iy / STRIP;
+    const int row = (strip & 1) ? N - 1 - ix : ix;
+    return (strip * N + row) * STRIP + iy % STRIP;
+}
+
 // Counts the particles of a wave into their cells and returns each one's
 // rank in its cell (arrival order): consecutive lanes with the same key (the
 // common case when particles are visited in cell order) add their number
@@ -124,7 +140,7 @@ __device__ __forceinline__ int count_rank(int *count, int key)
     return key >= 0 ? base + (lane - h) : -1;
 }
 
-// Bins a plasma particle for the deposit: returns its cell key ix N + iy and
+// Bins a plasma particle for the deposit: returns its cell_key and
 // writes its record at rec[j] (its binning position), or returns -1 (with an error bit) when the 5x5
 // stencil would leave the grid or the position is not finite.  P Q Z M qv are
 // the stored px py pz m q.
@@ -159,7 +175,7 @@ __device__ __forceinline__ int bin_particle(double x, double y, double h, int N,
     r.c2 = (TP)(Q * r_g);
     r.c3 = (TP)(Z * r_g);
     rec[j] = r;
-    return ix * N + iy;
+    return cell_key(ix, iy, N);
 }
 
 }  // namespace lc3d

@@ -71,12 +71,12 @@ __global__ __launch_bounds__(256) void k_bin(int64_t n, double h, int N,
         bs.key[k] = key;
         bs.pid[k] = (int)k;
     }
-    // Unbinned particles are counted (and ranked) in count[N * N].
-    const int r = count_rank(bs.count, k < n ? (key >= 0 ? key : N * N) : -1);
+    // Unbinned particles are counted (and ranked) in count[cell_keys(N)].
+    const int r = count_rank(bs.count, k < n ? (key >= 0 ? key : cell_keys(N)) : -1);
     if (k < n) bs.rank[k] = r;
 }
 
-// ---- exclusive scan of the N*N cell counts -----------------------------------------
+// ---- exclusive scan of the cell counts ---------------------------------------------
 // Inclusive scan of v over the wave's lanes in order (__shfl_up steps).
 __device__ __forceinline__ int wave_inclusive_scan(int v)
 {
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(GATHER_THREADS, GatherPlan<TP>::waves) void k_depos
         const int cx = X0 - 2 + t / H, cy = Y0 - 2 + t % H;
         int first = 0, n = 0, dsl = -1;
         if (cx >= 0 && cx < N && cy >= 0 && cy < N) {
-            const int cell = cx * N + cy;
+            const int cell = cell_key(cx, cy, N);
             first = start[cell];
             n = start[cell + 1] - first;
             dsl = bs.dslot[cell];
@@ -691,7 +691,7 @@ hipError_t launch_deposit(const PushGeom &g, const SortArrays<TP> &a, bool use_f
                           TG *ro1, TG *jx1, TG *jy1, TG *jz1, hipStream_t s, KernelTimer *timer)
 {
     const int N = g.N;
-    const int ncell = N * N;
+    const int ncell = cell_keys(N);
     const double *xo = use_full ? a.xo : a.xo_prev;
     const double *yo = use_full ? a.yo : a.yo_prev;
     const TP *px = use_full ? a.px : a.px_prev;

@@ -42,20 +42,20 @@ inline int scan_tiles(int64_t ncell) { return (int)((ncell + SCAN_TILE_CELLS) / 
 
 // Binning state shared by push and deposit (owned by the context).
 struct BinState {
-    int *count;       // N*N + 1, zero between deposits (the scan and the list
+    int *count;       // cell_keys(N) + 1, zero between deposits (the scan and the list
                       // sort clear them)
-    int *start;       // N*N + 1: each cell's list start (written by k_order_cells)
-    int *lstart;      // N*N + 1: each cell's list start within its scan tile
+    int *start;       // cell_keys(N) + 1: each cell's list start (written by k_order_cells)
+    int *lstart;      // cell_keys(N) + 1: each cell's list start within its scan tile
     int *base;        // per scan tile: the sum of the tiles before it (zero
                       // between deposits: the gather clears it)
-    int nbase;        // scan tiles, scan_tiles(N*N)
+    int nbase;        // scan tiles, scan_tiles(cell_keys(N))
     // key, rank, pid and rec are indexed by binning position: the thread
     // index j of the pass that binned the particle (the push visits particle
     // order[j], k_bin particle j).
     int *key;         // per position: cell index or -1
     int *rank;        // per position: its place among the particles counted into
                       // the same cell (or among the unbinned ones, counted in
-                      // count[N*N]), in arrival order
+                      // count[cell_keys(N)]), in arrival order
     int *pid;         // per position: the particle binned there
     int *pos;         // per list slot: binning positions sorted by cell (each
                       // cell's list ascending), then the unbinned ones
@@ -67,7 +67,7 @@ struct BinState {
     int *big;         // dense cells (more than 16 particles), in queue order
     int *nbig;        // how many cells `big` holds
     int bigcap;       // capacity of `big`
-    int *dslot;       // N*N: a cell's slot in `big`, or -1
+    int *dslot;       // cell_keys(N): a cell's slot in `big`, or -1
     void *dense;      // per dense cell: its 5 x 5 x 4 deposit (deposit.hip)
 };
 
@@ -142,23 +142,17 @@ hipError_t launch_move_wo_fields(int64_t n, double xi_step, const TP *m, double 
 
 // plasma3d/move.py:52-148.  first=true folds in the free-streaming estimate
 // from the previous layer (move.py:331-349); bin=true also records each
-// particle's deposit cell for the deposit that follows.  `order`, when not
+// particle's deposit cell for the deposit that follows; momenta=false leaves
+// px, py and pz of the particles it moves unwritten (an earlier push of a
+// step, whose momenta nothing reads).  `order`, when not
 // null, is a permutation of the n particles (the last deposit's cell order):
 // thread j pushes particle order[j], so neighbouring threads read
 // neighbouring field cells.  Each particle is pushed independently, so the
 // result does not depend on the order.
 template <typename TP, typename TF>
 hipError_t launch_push(const PushGeom &g, const Fields6<TF> &f, const SortArrays<TP> &a,
-                       bool first, bool bin, const BinState &bs, const int *order, hipStream_t s,
-                       KernelTimer *timer = nullptr);
-// The FP32-bulk push from float64 fields read as float32: the six fields are
-// first rounded into f32 (6 fields32_stride(N) floats), then pushed as
-// launch_push<float, float> does, both inside the push timing.
-inline int64_t fields32_stride(int N) { return ((int64_t)N * N + 3) & ~(int64_t)3; }
-hipError_t launch_push_f64_fields_as_f32(const PushGeom &g, const Fields6<double> &f,
-                                         float *f32, const SortArrays<float> &a, bool first,
-                                         bool bin, const BinState &bs, const int *order,
-                                         hipStream_t s, KernelTimer *timer = nullptr);
+                       bool first, bool bin, bool momenta, const BinState &bs, const int *order,
+                       hipStream_t s, KernelTimer *timer = nullptr);
 
 // plasma3d/weights.py:35-67, 249-285 for one sort.  When `binned` is false
 // the cells are computed here; otherwise the preceding push recorded them.

@@ -312,6 +312,41 @@ def test_push_matches_oracle(N, precision):
         assert e < bound, (k, e)
 
 
+@pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
+@pytest.mark.parametrize('n', [1, 255, 65535, 65536, 65537, 70000])
+def test_push_does_not_depend_on_how_particles_are_visited(n, precision):
+    """One smart push of n particles drawn from the lattice in random order
+    gives each of them the bits it gets when the whole lattice is pushed in
+    tiles (every particle's arithmetic is the same whatever its block reads
+    its fields from).  n lies on both sides of the particle number from which
+    blocks stage their fields in LDS; the drawn blocks' stencils span the
+    whole grid, so they read from memory; 65536 = 256^2 is square but no
+    lattice."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.move import get_plasma_particles_mover
+    print(f'scattered push n={n} {precision}', flush=True)
+    N, fineness = 129, 3
+    rng = np.random.default_rng(n)
+    lattice = _round_bulk(_random_plasma(rng, _params(N, fineness=fineness)))
+    pick = rng.permutation(lattice['m'].size)[:n]
+    drawn = {k: np.ascontiguousarray(v.ravel()[pick]) for k, v in lattice.items()}
+    bulk = torch.float32 if precision == 'fp32-bulk' else torch.float64
+    fields = Arrays.wrap(**{k: dev(0.2 * _smooth(rng, N), bulk)
+                            for k in ('Ex', 'Ey', 'Ez', 'Bx', 'By', 'Bz', 'Phi')})
+    wo, smart = get_plasma_particles_mover(_cfg(N, precision=precision, fineness=fineness))
+    const = Arrays.wrap()
+    const.sorts = {'electrons': 0}
+    out = []
+    for a in (lattice, drawn):
+        prev = {'electrons': _sort_arrays(a, bulk)}
+        out.append(smart(fields, prev, wo(prev, const), const)['electrons'])
+    torch.cuda.synchronize()
+    assert drawn['m'].size == n
+    for k in ('x_offt', 'y_offt', 'px', 'py', 'pz', 'q'):
+        whole, part = (host(getattr(o, k)).ravel() for o in out)
+        assert np.array_equal(whole[pick], part), k
+
+
 def _wall_plasma(rng, p):
     """A lattice whose outer particles are set up to cross the reflection
     boundary b = h (N/2 - 10).  With zero offsets and momenta
