@@ -134,6 +134,27 @@ uint64_t rfft_default_plan(int L)
     return packed;
 }
 
+// Default launch shape of the Stockham kernels: complex values of LDS and
+// transforms per block.  Few transforms a block, so that all of the chip's
+// CUs have blocks (7 (N + 1) / 2 transforms a kernel) and a CU holds several;
+// but two where a radix-16 stage of one (L / 16 butterflies) would leave most
+// of the 256 threads idle and the blocks still outnumber the CUs.  Short
+// transforms take the larger LDS size: the smaller one's kernels are compiled
+// for more waves a SIMD and spill.  Measured (default plan, us per solve,
+// this shape against filling the largest LDS size): float32 N = 129 29 (68),
+// 257 39 (76), 417 72 (97), 513 78 (101), 1025 278 (388); float64 129 32 (50),
+// 257 48 (59), 385 94 (101), 513 133, 1025 496.
+void rfft_default_shape(int L, bool f32, int &cap, int &tpb)
+{
+    if (f32) {
+        cap = L > 512 && L < 1024 ? 2048 : 4096;
+        tpb = L == 1024 ? 2 : 1;
+    } else {
+        cap = (L > 256 && L < 512) || (L > 640 && L < 1024) ? 2048 : 4096;
+        tpb = L == 512 || L == 1024 ? 2 : L > 512 && L <= 640 ? 4096 / (2 * L) : 1;
+    }
+}
+
 // Packs a caller's plan for the length-L FFT; 0 when it is not one.
 uint64_t rfft_pack_plan(int L, int ns, const int32_t *radix)
 {
@@ -464,8 +485,12 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
         } else {
             c->rf_stages = p->fft_nstages > 0 ? rfft_pack_plan(L, p->fft_nstages, p->fft_radix)
                                               : rfft_default_plan(L);
-            c->rf_cap = p->rfft_cap > 0 ? p->rfft_cap : (f32s ? 8192 : 4096);
-            c->rf_tpb = p->rfft_tpb > 0 ? p->rfft_tpb : c->rf_cap / (2 * L);
+            if (p->rfft_cap <= 0 && p->rfft_tpb <= 0) {
+                rfft_default_shape(L, f32s, c->rf_cap, c->rf_tpb);
+            } else {
+                c->rf_cap = p->rfft_cap > 0 ? p->rfft_cap : (f32s ? 8192 : 4096);
+                c->rf_tpb = p->rfft_tpb > 0 ? p->rfft_tpb : c->rf_cap / (2 * L);
+            }
             if (c->rf_stages == 0 || !rfft_cap_supported(f32s, c->rf_cap) || c->rf_tpb < 1 ||
                 2 * (int64_t)c->rf_tpb * L > c->rf_cap) {
                 delete c;
