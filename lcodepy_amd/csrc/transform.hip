@@ -20,6 +20,8 @@
 //               tiles through LDS, 16x16x4 matrix-core products; the last
 //               row and column by the blocks of the last tile row and
 //               column), optionally scaled by M;
+//   k_gemm_split the same in float64 for the smaller N (16 x 16 or 32 x 32
+//               tiles, k split over the waves);
 //   k_assemble  outputs (full / half fields) and the Bz row sums;
 //   k_bz_finalize  mean of Bz removed, half-step Bz.
 #include "mfma.h"
@@ -51,6 +53,9 @@ __global__ __launch_bounds__(256) void k_rhs(RhsEval<TG, TPRED> rhs, TG *__restr
 }
 
 constexpr int GBM = 64, GBN = 64;   // output tile
+// The float64 product: 16 x 16 split tiles below GEMM_SMALL, 32 x 32 split
+// tiles below GEMM_SPLIT, k_gemm_mfma from there on (k_gemm_split).
+constexpr int GEMM_SMALL = 200, GEMM_SPLIT = 336;
 constexpr int GTJ = GBN / 32;       // 16-column products per wave (waves 2 x 2)
 // Depth of a k tile: 64 in float32, 32 in float64 (two blocks per CU fit
 // the double-buffered LDS tiles either way).
@@ -246,11 +251,127 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(GemmBatch<T> bt, int N, Sc
     }
 }
 
+// The float64 product, with the k range split over the waves of a block: the
+// tile is (16 R) x (16 R) output elements, and wave w sums k in its quarter of
+// [0, N) for the whole tile, its operands straight from memory into the
+// matrix cores' registers (the next 16 k in flight), so that nothing waits at
+// a barrier before the four partial tiles meet in LDS.  The 64 x 64 tiles of
+// k_gemm_mfma give N = 129 28 blocks and N = 321 175, each a serial chain of k
+// tiles; float32 keeps them, where the order of the k sum decides the result
+// at its precision.  Measured per solve (four products and the passes around
+// them; 16 x 16 split, 32 x 32 split, k_gemm_mfma; us): N = 65 26, 30, 53; 129
+// 36, 39, 73; 193 57, 62, 98; 225 77, 68, 97; 257 92, 91, 115; 321 161, 134, 140;
+// 385 247, 189, 169; 513 482, 333, 293: the split tiles read (N / 16 R)^2 N of
+// both operands past the L2 at about 6.8 TB/s, which bounds them from N of
+// about 300.
+// Lane l of a wave takes k = kk + 4 (l / 16) + s in step s of a group of 16, the
+// same for A and B, so that it reads four neighbouring elements of A's row.
+// Rows, columns and k beyond the matrix read its last ones and count zero.
+template <typename T, int R, bool SCALE>
+__global__ __launch_bounds__(256) void k_gemm_split(GemmBatch<T> bt, int N, ScaleGeom sg)
+{
+    using MM = Mfma16<T>;
+    using acc_t = typename MM::acc_t;
+    constexpr int TS = 16 * R;
+    __shared__ T red[4][TS][TS + 1];
+    // Consecutive tiles of a field on one XCD: they share rows of A, and B.
+    const int tiles = (N + TS - 1) / TS;
+    const int id = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int f = id / (tiles * tiles), tile = id % (tiles * tiles);
+    const int row0 = tile / tiles * TS, col0 = tile % tiles * TS;
+    const T *__restrict__ A = bt.A[f];
+    const T *__restrict__ B = bt.B[f];
+    T *__restrict__ C = bt.C[f];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, li = lane % 16, lk = lane / 16;
+    const int share = ((N + 15) / 16 + 3) / 4 * 16;   // k of a wave
+    const int k0 = min(N, wave * share), k1 = min(N, k0 + share);
+
+    const T *pa[R];
+    const T *pb[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        pa[r] = A + (size_t)min(row0 + 16 * r + li, N - 1) * N;
+        pb[r] = B + min(col0 + 16 * r + li, N - 1);
+    }
+    acc_t acc[R][R];
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = T(0);
+    T a[2][R][4], b[2][R][4];
+    auto load = [&](auto set, int kk) {
+        constexpr int S = decltype(set)::value;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int k = kk + 4 * lk + s, kc = min(k, N - 1);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                a[S][r][s] = pa[r][kc];
+                b[S][r][s] = pb[r][(size_t)kc * N];
+            }
+            if (k >= k1) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) a[S][r][s] = b[S][r][s] = T(0);
+            }
+        }
+    };
+    auto multiply = [&](auto set) {
+        constexpr int S = decltype(set)::value;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int j = 0; j < R; ++j) acc[i][j] = MM::mma(a[S][i][s], b[S][j][s], acc[i][j]);
+    };
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    if (k0 < k1) {   // whole waves
+        load(Zero{}, k0);
+        for (int kk = k0; kk < k1; kk += 32) {
+            if (kk + 16 < k1) load(One{}, kk + 16);
+            multiply(Zero{});
+            if (kk + 32 < k1) load(Zero{}, kk + 32);
+            if (kk + 16 < k1) multiply(One{});
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                red[wave][16 * i + MM::row(lk, r)][16 * j + li] = acc[i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int e = threadIdx.x; e < TS * TS; e += 256) {
+        const int i = e / TS, j = e % TS, gr = row0 + i, gc = col0 + j;
+        if (gr < N && gc < N) {
+            T v = (red[0][i][j] + red[1][i][j]) + (red[2][i][j] + red[3][i][j]);
+            if (SCALE) v = (T)((double)v * solver_factor(f, gr, gc, N, sg));
+            C[(size_t)gr * N + gc] = v;
+        }
+    }
+}
+
+template <typename T, int R, bool SCALE>
+void gemm_split_launch(const GemmBatch<T> &bt, int N, const ScaleGeom &sg, hipStream_t s)
+{
+    const int tiles = (N + 16 * R - 1) / (16 * R);
+    k_gemm_split<T, R, SCALE><<<7 * tiles * tiles, 256, 0, s>>>(bt, N, sg);
+}
+
 template <typename T, bool SCALE>
 void gemm_launch(const GemmBatch<T> &bt, int N, const ScaleGeom &sg, hipStream_t s)
 {
     static_assert(GemmTile<T>::BK <= 64, "the edge loaders use threads 0..127");
     static_assert(GBN % 32 == 0 && GBN <= 64 && GBM == 64, "wave layout 2 x 2");
+    if constexpr (std::is_same<T, double>::value) {
+        if (N < GEMM_SMALL) return gemm_split_launch<T, 1, SCALE>(bt, N, sg, s);
+        if (N < GEMM_SPLIT) return gemm_split_launch<T, 2, SCALE>(bt, N, sg, s);
+    }
     const dim3 grid((N - 1 + GBN - 1) / GBN, (N - 1 + GBM - 1) / GBM, 7);
     k_gemm_mfma<T, SCALE><<<grid, 256, 0, s>>>(bt, N, sg);
 }

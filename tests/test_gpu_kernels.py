@@ -136,6 +136,14 @@ def test_compute_fields_matches_oracle(N, precision, solver, extra=None):
     print(f'compute_fields N={N} {precision} {solver}: worst {worst:.1e}')
 
 
+@pytest.mark.parametrize('N', [9, 17, 199, 201, 335, 337])
+def test_float64_matrix_solve_at_the_edges_of_its_tiles(N):
+    """The float64 transform products at both sides of each size where
+    another tile takes over, at one more than a multiple of 16, and at the
+    smallest grid."""
+    test_compute_fields_matches_oracle(N, 'fp64', 'matrix')
+
+
 @pytest.mark.parametrize('N,precision,plan,cap,tpb', [
     (513, 'fp64', (2,) * 10, 2048, 1),
     (513, 'fp64', (4, 4, 4, 4, 4), 4096, 1),
