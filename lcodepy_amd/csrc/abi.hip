@@ -26,7 +26,7 @@ struct lc3d_ctx {
     int64_t cap = 0;
     FftPlan plan{};
     // binning
-    int *count = nullptr, *start = nullptr, *lstart = nullptr, *base = nullptr, *key = nullptr;
+    int *count = nullptr, *lstart = nullptr, *base = nullptr, *key = nullptr;
     int *idx = nullptr, *rank = nullptr, *pid = nullptr, *pos = nullptr;
     int nbase = 0;
     unsigned *err = nullptr;
@@ -184,10 +184,9 @@ PushGeom push_geom(const lc3d_ctx *c, int64_t n)
 BinState bin_state(const lc3d_ctx *c, int col)
 {
     const int64_t cap = std::max<int64_t>(1, c->cap);
-    return BinState{c->count, c->start,  c->lstart, c->base,   c->nbase,
-                    c->key,   c->rank,   c->pid,    c->pos,    c->idx + col * cap,
-                    c->err,   c->rec,    cap,       c->big,    c->nbig,
-                    c->bigcap, c->dslot, c->dense};
+    return BinState{c->count, c->lstart, c->base, c->nbase, c->key,  c->rank,   c->pid,
+                    c->pos,   c->idx + col * cap, c->err,  c->rec,  cap,      c->big,
+                    c->nbig,  c->bigcap, c->dslot, c->dense};
 }
 
 template <typename TP> SortArrays<TP> sort_arrays(const lc3d_sort *s)
@@ -533,7 +532,6 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
     const size_t tg = f32 ? sizeof(float) : sizeof(double);
     const size_t cap = (size_t)std::max<int64_t>(1, c->cap);
     bool ok = hipMalloc(&c->count, (nkeys + 1) * sizeof(int)) == hipSuccess &&
-              hipMalloc(&c->start, (nkeys + 1) * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->lstart, (nkeys + 1) * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->base, nblocks * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->key, cap * sizeof(int)) == hipSuccess &&
@@ -640,7 +638,6 @@ void lc3d_destroy(lc3d_ctx *c)
         for (hipEvent_t &e : c->timer.ev) (void)hipEventDestroy(e);
     }
     (void)hipFree(c->count);
-    (void)hipFree(c->start);
     (void)hipFree(c->lstart);
     (void)hipFree(c->base);
     (void)hipFree(c->key);

@@ -117,6 +117,15 @@ __device__ __forceinline__ int cell_key(int ix, int iy, int N) {
     return (strip * N + row) * STRIP + iy % STRIP;
 }
 
+// Called by every thread of a binning pass: its first block empties what the
+// scan that follows adds to.
+__device__ __forceinline__ void clear_scan(const BinState &bs)
+{
+    if (blockIdx.x != 0) return;
+    for (int i = threadIdx.x; i < bs.nbase; i += blockDim.x) bs.base[i] = 0;
+    if (threadIdx.x == 0) *bs.nbig = 0;
+}
+
 // Counts the particles of a wave into their cells and returns each one's
 // rank in its cell (arrival order): consecutive lanes with the same key (the
 // common case when particles are visited in cell order) add their number

@@ -42,12 +42,11 @@ inline int scan_tiles(int64_t ncell) { return (int)((ncell + SCAN_TILE_CELLS) / 
 
 // Binning state shared by push and deposit (owned by the context).
 struct BinState {
-    int *count;       // cell_keys(N) + 1, zero between deposits (the scan and the list
-                      // sort clear them)
-    int *start;       // cell_keys(N) + 1: each cell's list start (written by k_order_cells)
+    int *count;       // cell_keys(N) + 1, zero between deposits (the scan and the
+                      // scatter clear them)
     int *lstart;      // cell_keys(N) + 1: each cell's list start within its scan tile
-    int *base;        // per scan tile: the sum of the tiles before it (zero
-                      // between deposits: the gather clears it)
+    int *base;        // per scan tile: the sum of the tiles before it (the
+                      // binning pass clears it)
     int nbase;        // scan tiles, scan_tiles(cell_keys(N))
     // key, rank, pid and rec are indexed by binning position: the thread
     // index j of the pass that binned the particle (the push visits particle
@@ -57,8 +56,8 @@ struct BinState {
                       // the same cell (or among the unbinned ones, counted in
                       // count[cell_keys(N)]), in arrival order
     int *pid;         // per position: the particle binned there
-    int *pos;         // per list slot: binning positions sorted by cell (each
-                      // cell's list ascending), then the unbinned ones
+    int *pos;         // per list slot: binning positions sorted by cell (within
+                      // a cell by rank), then the unbinned ones
     int *idx;         // per list slot: the particle ids of pos (the cell order
                       // the next push of this sort visits)
     unsigned *err;    // sticky error bits
@@ -67,7 +66,7 @@ struct BinState {
     int *big;         // dense cells (more than 16 particles), in queue order
     int *nbig;        // how many cells `big` holds
     int bigcap;       // capacity of `big`
-    int *dslot;       // cell_keys(N): a cell's slot in `big`, or -1
+    int *dslot;       // cell_keys(N): a dense cell's slot in `big`
     void *dense;      // per dense cell: its 5 x 5 x 4 deposit (deposit.hip)
 };
 

@@ -136,6 +136,7 @@ __global__ __launch_bounds__(STAGED ? PUSH_THREADS : PUSH_FEW_THREADS,
     __shared__ FieldPair<TP> s_f[3][STAGED ? PUSH_WINDOW : 1];
     __shared__ float s_red[PUSH_THREADS / 64][4];
     constexpr int THREADS = STAGED ? PUSH_THREADS : PUSH_FEW_THREADS;
+    if (BIN) clear_scan(bs);
     // Consecutive blocks of the order go to the same XCD, so each XCD's L2
     // fetches the field rows of its own stretch of cells.
     const int block = xcd_swizzle(blockIdx.x, gridDim.x);

@@ -85,6 +85,14 @@ inline int __shfl(int v, int src) {
     emu_sync_wave();
     return r;
 }
+inline double __shfl(double v, int src) {
+    int t = threadIdx.x, w = t / 64;
+    emu_shfl_d[t] = v;
+    emu_sync_wave();
+    double r = emu_shfl_d[(src & 63) + w * 64];
+    emu_sync_wave();
+    return r;
+}
 inline unsigned long long __ballot(int pred) {
     int t = threadIdx.x, w = t / 64;
     emu_shfl_i[t] = pred != 0;
