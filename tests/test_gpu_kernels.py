@@ -245,6 +245,46 @@ def test_deposit_matches_oracle_and_is_deterministic(N, precision):
         assert not torch.any(u[1])
 
 
+@pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
+@pytest.mark.parametrize('N', [65, 433, 449])
+def test_deposit_of_cells_at_the_edges_of_the_lists(N, precision):
+    """Cells of 0, 1, 4, 8, 9, 15, 16, 17 and 18 particles (each list length at
+    which the gather ranks a list otherwise, and both sides of a dense cell),
+    with a band of rows that hold 16 in every cell (no two fit the staging
+    together), visited in random order, at a grid that takes tiles of four rows
+    and on both sides of where eight begin.  A density sums up to 25 x 18 terms
+    of about 30 roundings each, of which a tenth may be left by cancellation:
+    1e-12 of the maximum in float64, 3e-5 in float32."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.weights import get_deposit_plasma
+    print(f'list edges N={N} {precision}', flush=True)
+    f32 = precision == 'fp32-bulk'
+    rng = np.random.default_rng(N)
+    fineness = 5
+    p = _params(N, fineness=fineness)
+    count = np.zeros((N, N), dtype=int)
+    inner = slice(8, N - 8)
+    count[inner, inner] = rng.choice([0, 1, 4, 8, 9, 15, 16, 17, 18], (N - 16, N - 16))
+    count[20:26, inner] = 16
+    cell = rng.permutation(np.repeat(np.arange(N * N), count.ravel()))
+    n = cell.size
+    at = lambda k: (k - N // 2 + 0.98 * rng.uniform(-0.5, 0.5, n)) * p.h
+    m = np.full(n, 0.01)
+    a = dict(x_init=at(cell // N), y_init=at(cell % N), x_offt=np.zeros(n), y_offt=np.zeros(n),
+             q=-m, m=m, **{k: m * rng.normal(0, 0.1, n) for k in ('px', 'py', 'pz')})
+    if f32:
+        a = _round_bulk(a)
+    g = [np.zeros((N, N)) for _ in range(4)]
+    O.deposit_sort(p, a, *g)
+    deposit = get_deposit_plasma(_cfg(N, precision=precision, fineness=fineness))
+    const = Arrays.wrap()
+    const.sorts = {'electrons': 0}
+    out = deposit({'electrons': _sort_arrays(a, torch.float32 if f32 else torch.float64)}, const)
+    torch.cuda.synchronize()
+    for u, w in zip(out, g):
+        assert relerr(host(u[0]), w) < (3e-5 if f32 else 1e-12)
+
+
 @pytest.mark.parametrize('N,frac', [(65, 0.005), (65, 0.05), (65, 0.3), (129, 0.45)])
 def test_deposit_of_collapsed_plasma(N, frac):
     """A fraction of the particles collapsed into the cell on the axis
