@@ -15,6 +15,7 @@
  *   lc3d_layout_beam_layer beam3d/beam_calculator.py:82-93 (layout_beam_layer)
  *   lc3d_beam_substep     beam3d/beam_calculator.py:97-114 (start_moving_layer)
  *   lc3d_move_beam        beam3d/move.py:294-309     (move_beam_particles)
+ *   lc3d_beam_advance     beam3d/beam_calculator.py:97-143 (one layer)
  *   lc3d_energy_flux      diagnostics/FXi/Strategy3D.py:6-25 (calculate_energy_fluxes)
  *   lc3d_probe_sample     diagnostics/FXi/Strategy3D.py:59-82 (the f(xi) probe values)
  *   lc3d_abs_max          diagnostics/FXi/Strategy3D.py:84-95 (process_chaotic*)
@@ -283,6 +284,31 @@ int lc3d_move_beam(lc3d_ctx *ctx, int64_t n, int64_t beam_layer_idx, const doubl
 int lc3d_beam_split(lc3d_ctx *ctx, int64_t n, int32_t nf, int32_t ni, const double *f,
                     const int64_t *iv, const uint8_t *flags, double *out_f, int64_t *out_i,
                     int64_t *counts, void *stream);
+/* A range of n columns of packed beam rows: float64 row r of column c (xi x y
+ * px py pz q_m q_norm dt) at f[r * f_stride + c], int64 row r (id,
+ * remaining_steps) at i[r * i_stride + c]. */
+typedef struct lc3d_beam_rows {
+    int64_t n;
+    const double *f;
+    int64_t f_stride;
+    const int64_t *i;
+    int64_t i_stride;
+} lc3d_beam_rows;
+
+/* Bytes of scratch lc3d_beam_advance needs for n particles. */
+#define LC3D_BEAM_ADVANCE_SCRATCH(n) (89 * (int64_t)(n) + 12 * (((int64_t)(n) + 31) / 32))
+
+/* One layer of beam_calculator.py:97-143 in one call: lc3d_beam_substep of the
+ * layer's particles, lc3d_move_beam of the layer followed by the particles
+ * that fell into it, and lc3d_beam_split of the result into out_f (3 x 9 x n),
+ * out_i (3 x 2 x n) and counts (device int64[3]), n = layer->n + fell->n.  The
+ * rows read are not changed.  scratch: 8-byte aligned device memory of at least
+ * LC3D_BEAM_ADVANCE_SCRATCH(n) bytes.  Nothing is done when n is 0. */
+int lc3d_beam_advance(lc3d_ctx *ctx, const lc3d_beam_rows *layer, const lc3d_beam_rows *fell,
+                      int64_t beam_layer_idx, double substepping_energy, double time_step,
+                      const lc3d_fields6 *fields_k, const lc3d_fields6 *fields_k1, void *scratch,
+                      int64_t scratch_bytes, double *out_f, int64_t *out_i, int64_t *counts,
+                      void *stream);
 /* Total energy flux of a plasma layer, diagnostics/FXi/Strategy3D.py:6-25
  * (calculate_energy_fluxes): the sum over the grid of (Ez^2 + Bz^2 +
  * (Ex - By)^2 + (Ey + Bx)^2) h^2 / 2 plus the sum over the n electrons of

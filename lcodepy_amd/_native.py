@@ -90,6 +90,11 @@ class ProbeSources(ctypes.Structure):
                 ('is_f32', ctypes.c_int32 * PROBE_MAX_SOURCES)]
 
 
+class BeamRows(ctypes.Structure):
+    _fields_ = [('n', ctypes.c_int64), ('f', _vp), ('f_stride', ctypes.c_int64), ('i', _vp),
+                ('i_stride', ctypes.c_int64)]
+
+
 class Sort(ctypes.Structure):
     _fields_ = [('n', ctypes.c_int64),
                 ('x_init', _vp), ('y_init', _vp), ('m', _vp),
@@ -108,7 +113,7 @@ SYMBOLS = ('lc3d_create', 'lc3d_destroy', 'lc3d_last_error', 'lc3d_precision',
            'lc3d_layout_beam_layer',
            'lc3d_beam_substep', 'lc3d_move_beam', 'lc3d_energy_flux', 'lc3d_probe_sample',
            'lc3d_abs_max', 'lc3d_energy_flux_noalloc', 'lc3d_autotune_solve',
-           'lc3d_noise_filter', 'lc3d_beam_split')
+           'lc3d_noise_filter', 'lc3d_beam_split', 'lc3d_beam_advance')
 
 _LIB = None
 _LOCK = threading.Lock()
@@ -149,6 +154,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
                                       P(i32)]
     L.lc3d_noise_filter.argtypes = [_vp, P(Sort), _vp]
     L.lc3d_beam_split.argtypes = [_vp, i64, i32, i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp]
+    L.lc3d_beam_advance.argtypes = [_vp, P(BeamRows), P(BeamRows), i64, dbl, dbl, P(Fields6),
+                                    P(Fields6), _vp, i64, _vp, _vp, _vp, _vp]
     L.lc3d_probe_sample.argtypes = [_vp, P(ProbeSources), i32, _vp, _vp, _vp, _vp]
     L.lc3d_abs_max.argtypes = [_vp, _vp, i64, i64, i64, i64, i64, i64, _vp, _vp]
     L.lc3d_move_beam.argtypes = [_vp, i64, i64, _vp, _vp, P(Fields6), P(Fields6), _vp, _vp,

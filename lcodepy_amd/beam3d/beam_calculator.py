@@ -1,9 +1,12 @@
 """Beam layer calculators (beam3d/beam_calculator.py:60-181)."""
 from __future__ import annotations
 
+import ctypes
+
 from .. import runtime
-from .._native import ptr, stream_ptr
+from .._native import BeamRows, ptr, stream_ptr
 from ..config import Config
+from ..plasma3d import _bind
 from .data import BeamParticles, empty_rounded
 from .move import get_move_beam_particles
 from .weights import get_deposit_beam
@@ -97,9 +100,52 @@ class BeamCalculator:
         done.record()
         return PendingMove(out_f, out_i, counts, done)
 
+    def advance_layer_async(self, layer: BeamParticles, fell: BeamParticles, pl_layer_idx,
+                            fields_after_layer, fields_before_layer) -> 'PendingMove':
+        """:meth:`move_beam_layer_async` of ``layer`` followed by the particles
+        ``fell`` into it, in one library call that reads both where they are
+        (column slices of packed rows included) and changes neither."""
+        import torch
+        n, dev = layer.size + fell.size, runtime.device()
+        if n == 0:
+            return PendingMove(None, None, None, None)
+        for f in (fields_after_layer, fields_before_layer):
+            if f.Ex.dtype.itemsize != 8:
+                raise TypeError('the beam moves in the float64 fields of layers k and k+1')
+        scratch_bytes = 89 * n + 12 * ((n + 31) // 32)    # LC3D_BEAM_ADVANCE_SCRATCH
+        scratch = empty_rounded((scratch_bytes,), torch.uint8, dev)
+        out_f = empty_rounded((3, 9, n), torch.float64, dev)
+        out_i = empty_rounded((3, 2, n), torch.int64, dev)
+        counts_dev = torch.empty(3, dtype=torch.int64, device=dev)
+        rows = [_beam_rows(b) for b in (layer, fell)]
+        self.ctx.check(self.ctx.lib.lc3d_beam_advance(
+            self.ctx.handle, rows[0], rows[1], int(pl_layer_idx) - 1, self.substep_energy,
+            self.time_step, _bind.fields6(fields_after_layer), _bind.fields6(fields_before_layer),
+            scratch.data_ptr(), scratch_bytes, out_f.data_ptr(), out_i.data_ptr(),
+            counts_dev.data_ptr(), stream_ptr()), 'lc3d_beam_advance')
+        counts = torch.empty(3, dtype=torch.int64, pin_memory=True)
+        counts.copy_(counts_dev, non_blocking=True)
+        done = torch.cuda.Event()
+        done.record()
+        return PendingMove(out_f, out_i, counts, done)
+
     def create_next_layer(self, beam_layer_to_layout, fell_to_next_layer, ro_beam_full):
         beam_layer_to_move = BeamParticles().append(beam_layer_to_layout).append(fell_to_next_layer)
         return beam_layer_to_move, fell_to_next_layer.size, ro_beam_full.clone()
+
+
+def _beam_rows(b: BeamParticles) -> BeamRows:
+    """The packed rows of a layer as they are; rows whose columns are not
+    neighbours are copied first."""
+    if b.size == 0:
+        return BeamRows(0, None, 0, None, 0)
+    f, i = b.f, b.i
+    if f.stride(1) != 1 or i.stride(1) != 1:
+        b.contiguous()
+        f, i = b.f, b.i
+    if not (f.is_cuda and i.is_cuda) or f.dtype.itemsize != 8 or i.dtype.itemsize != 8:
+        raise TypeError('a beam layer is float64 and int64 rows on the device')
+    return BeamRows(f.shape[1], f.data_ptr(), f.stride(0), i.data_ptr(), i.stride(0))
 
 
 class PendingMove:

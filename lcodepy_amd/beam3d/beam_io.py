@@ -30,9 +30,8 @@ class BeamSource:
         xi_min = -self.xi_step_size * plasma_layer_idx
         xi_max = -self.xi_step_size * (plasma_layer_idx + 1)
         rest = self._neg_xi[self._offset:]
-        n = int(np.searchsorted(rest, -xi_max, side='right')
-                - np.searchsorted(rest, -xi_min, side='right'))
-        n = max(n, 0)
+        below, above = np.searchsorted(rest, (-xi_max, -xi_min), side='right')
+        n = max(int(below) - int(above), 0)
         layer = self.beam.slice(self._offset, self._offset + n)
         self._offset += n
         return layer

@@ -43,18 +43,22 @@ def _row_property(store: str, row: int):
 
 class BeamParticles:
     def __init__(self, xp=None, f=None, i=None):
-        import torch
-        from ..runtime import device
-        self.xp = torch
         if f is None:
+            import torch
+            from ..runtime import device
             dev = device()
             f = torch.zeros(len(FLOAT_KEYS), 0, dtype=torch.float64, device=dev)
             i = torch.zeros(len(INT_KEYS), 0, dtype=torch.int64, device=dev)
         self.f, self.i = f, i
 
     @property
+    def xp(self):
+        import torch
+        return torch
+
+    @property
     def size(self) -> int:
-        return int(self.f.shape[1])
+        return self.f.shape[1]
 
     @property
     def particles(self) -> np.ndarray:

@@ -914,6 +914,41 @@ int lc3d_beam_split(lc3d_ctx *c, int64_t n, int32_t nf, int32_t ni, const double
     return LC3D_OK;
 }
 
+int lc3d_beam_advance(lc3d_ctx *c, const lc3d_beam_rows *layer, const lc3d_beam_rows *fell,
+                      int64_t beam_layer_idx, double e_sub, double time_step,
+                      const lc3d_fields6 *fk, const lc3d_fields6 *fk1, void *scratch,
+                      int64_t scratch_bytes, double *out_f, int64_t *out_i, int64_t *counts,
+                      void *stream)
+{
+    auto rows_ok = [](const lc3d_beam_rows *r) {
+        return r && r->n >= 0 && r->n <= 0x3fffffff &&
+               (r->n == 0 || (r->f && r->i && r->f_stride >= r->n && r->i_stride >= r->n));
+    };
+    auto fields_ok6 = [](const lc3d_fields6 *f) {
+        return f && f->Ex && f->Ey && f->Ez && f->Bx && f->By && f->Bz;
+    };
+    if (!c || !rows_ok(layer) || !rows_ok(fell) || !fields_ok6(fk) || !fields_ok6(fk1))
+        return fail(c, LC3D_EINVAL, "beam_advance: bad arguments");
+    const int64_t n = layer->n + fell->n;
+    if (n == 0) return LC3D_OK;
+    if (!scratch || (uintptr_t)scratch % 8 != 0 || scratch_bytes < LC3D_BEAM_ADVANCE_SCRATCH(n) ||
+        !out_f || !out_i || !counts)
+        return fail(c, LC3D_EINVAL, "beam_advance: bad scratch or outputs");
+    const BeamGeom g{c->N, c->prm.grid_step_size, c->prm.xi_step_size, c->prm.lost_radius};
+    const BeamRows rl{layer->n, layer->f, layer->f_stride, layer->i, layer->i_stride};
+    const BeamRows rf{fell->n, fell->f, fell->f_stride, fell->i, fell->i_stride};
+    BeamScratch sc;
+    sc.f = static_cast<double *>(scratch);
+    sc.i = reinterpret_cast<int64_t *>(sc.f + 9 * n);
+    sc.count = reinterpret_cast<int *>(sc.i + 2 * n);
+    sc.group = reinterpret_cast<uint8_t *>(sc.count + 3 * ((n + 31) / 32));
+    hipError_t e = launch_beam_advance(g, rl, rf, beam_layer_idx, e_sub, time_step, f6<double>(fk),
+                                       f6<double>(fk1), sc, out_f, out_i, counts, c->err,
+                                       static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(c, e, "beam_advance");
+    return LC3D_OK;
+}
+
 int lc3d_energy_flux(lc3d_ctx *c, const lc3d_fields6 *f, int64_t n, const void *m,
                      const void *px, const void *py, const double *pz, double *psi, void *stream)
 {

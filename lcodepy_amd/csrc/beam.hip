@@ -50,9 +50,12 @@ __device__ __forceinline__ void fixed_add(unsigned long long *l0, unsigned long 
         q1 = -q1;
         q2 = -q2;
     }
-    atomicAdd(l0, (unsigned long long)q0);
-    atomicAdd(l1, (unsigned long long)q1);
-    atomicAdd(l2, (unsigned long long)q2);
+    // The taps of a layer's core meet in a few hundred cells, whose atomics
+    // are the deposit's time; a zero limb (the top one of every charge below
+    // 2^4) needs none.
+    if (q0 != 0) atomicAdd(l0, (unsigned long long)q0);
+    if (q1 != 0) atomicAdd(l1, (unsigned long long)q1);
+    if (q2 != 0) atomicAdd(l2, (unsigned long long)q2);
 }
 
 // The float64 nearest (up to two roundings) to the limb sums' value times
@@ -161,24 +164,6 @@ __global__ __launch_bounds__(256) void k_beam_finalize(int64_t nn, double h2,
     }
 }
 
-// beam3d/beam_calculator.py:18-34, 97-123: dt multiplier halved until
-// below sqrt(sqrt(1/q_m^2 + pz^2) / E_sub); dt = mult * time_step and
-// remaining_steps = int(1 / mult).
-__global__ __launch_bounds__(256) void k_beam_substep(int64_t n, const double *__restrict__ q_m,
-                                                      const double *__restrict__ pz, double e_sub,
-                                                      double time_step, double *__restrict__ dt,
-                                                      int64_t *__restrict__ steps)
-{
-    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double max_dt = sqrt(sqrt(1 / (q_m[k] * q_m[k]) + pz[k] * pz[k]) / e_sub);
-    double d = 1.0;
-    // At most 2^-40: the push below also caps its substep loop.
-    for (int it = 0; it < 40 && d > max_dt; ++it) d /= 2.0;
-    dt[k] = d * time_step;
-    steps[k] = (int64_t)(1. / d);
-}
-
 // This lane's share of the two-layer field gather of beam3d/move.py:70-91
 // (taps lane, lane + BEAM_LANES, ...), summed over the particle's lanes.
 template <typename TF>
@@ -210,30 +195,56 @@ __device__ __forceinline__ void gather2(const Fields6<TF> &a, const Fields6<TF> 
     }
 }
 
-// beam3d/move.py:31-127 (the CPU scheme; its trailing "fell" test compares
-// x, not xi, as move.py:123 does).
-// A group of BEAM_LANES lanes per particle; all lanes of a group run the
-// same substep loop (the same particle state), so the group's shuffles see
-// every lane of it; lane 0 writes the particle back.
-template <typename TF>
-__global__ __launch_bounds__(BEAM_THREADS) void k_beam_move(
-    BeamGeom g, int64_t n, double xi_k, double xi_k1, const double *__restrict__ q_m,
-    const double *__restrict__ dt, Fields6<TF> fk, Fields6<TF> fk1, int64_t *__restrict__ steps,
-    int64_t *__restrict__ id, double *__restrict__ x, double *__restrict__ y,
-    double *__restrict__ xi, double *__restrict__ px, double *__restrict__ py,
-    double *__restrict__ pz, uint8_t *__restrict__ lost, uint8_t *__restrict__ moved,
-    uint8_t *__restrict__ fell, unsigned *err)
+// beam3d/beam_calculator.py:18-34, 97-123: dt multiplier halved until
+// below sqrt(sqrt(1/q_m^2 + pz^2) / E_sub); dt = mult * time_step and
+// remaining_steps = int(1 / mult).
+__device__ __forceinline__ void substeps_of(double q_m, double pz, double e_sub, double time_step,
+                                            double &dt, int64_t &steps)
 {
-    const int64_t t = blockIdx.x * (int64_t)BEAM_THREADS + threadIdx.x;
-    const int64_t k = t / BEAM_LANES;
-    const int lane = (int)(t % BEAM_LANES);
-    if (k >= n) return;   // whole groups: n particles fill BEAM_LANES n lanes
+    const double max_dt = sqrt(sqrt(1 / (q_m * q_m) + pz * pz) / e_sub);
+    double d = 1.0;
+    // At most 2^-40: the push below also caps its substep loop.
+    for (int it = 0; it < 40 && d > max_dt; ++it) d /= 2.0;
+    dt = d * time_step;
+    steps = (int64_t)(1. / d);
+}
+
+__global__ __launch_bounds__(256) void k_beam_substep(int64_t n, const double *__restrict__ q_m,
+                                                      const double *__restrict__ pz, double e_sub,
+                                                      double time_step, double *__restrict__ dt,
+                                                      int64_t *__restrict__ steps)
+{
+    const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    double d;
+    int64_t rs;
+    substeps_of(q_m[k], pz[k], e_sub, time_step, d, rs);
+    dt[k] = d;
+    steps[k] = rs;
+}
+
+// One beam particle of a layer being moved.
+struct BeamState {
+    double x, y, xi, px, py, pz;
+    int64_t steps;
+    bool lost, fell, off;
+};
+
+// beam3d/move.py:31-127 (the CPU scheme; its trailing "fell" test compares
+// x, not xi, as move.py:123 does), by the BEAM_LANES lanes of the particle's
+// group, which all run the same substep loop, so that the group's shuffles
+// see every lane of it.
+template <typename TF>
+__device__ __forceinline__ void move_particle(const BeamGeom &g, double xi_k, double xi_k1,
+                                              double qm, double d, const Fields6<TF> &fk,
+                                              const Fields6<TF> &fk1, int lane, BeamState &b)
+{
     const int N = g.N;
     const double r2 = g.lost_radius * g.lost_radius;
-    const double qm = q_m[k], iqm = 1 / qm, d = dt[k];
+    const double iqm = 1 / qm;
     const double sgn = qm < 0 ? -1.0 : (qm > 0 ? 1.0 : 0.0);
-    double X = x[k], Y = y[k], XI = xi[k], PX = px[k], PY = py[k], PZ = pz[k];
-    int64_t rs = steps[k];
+    double X = b.x, Y = b.y, XI = b.xi, PX = b.px, PY = b.py, PZ = b.pz;
+    int64_t rs = b.steps;
     bool is_lost = false, is_fell = false, off = false;
     // Substep counts come from the caller; cap the loop so that a corrupt
     // count cannot keep the wave running (flagged as an error).
@@ -288,20 +299,170 @@ __global__ __launch_bounds__(BEAM_THREADS) void k_beam_move(
         }
         rs -= 1;
     }
-    if (off) atomicOr(err, ERR_BEAM_OFF_GRID);
-    if (lane != 0) return;
     if (rs == 0 && xi_k1 > X) is_fell = true;
-    if (is_lost) id[k] = -id[k];
-    x[k] = X;
-    y[k] = Y;
-    xi[k] = XI;
-    px[k] = PX;
-    py[k] = PY;
-    pz[k] = PZ;
-    steps[k] = rs;
-    lost[k] = is_lost;
-    fell[k] = is_fell;
-    moved[k] = !is_fell && !is_lost;
+    b = BeamState{X, Y, XI, PX, PY, PZ, rs, is_lost, is_fell, off};
+}
+
+// A group of BEAM_LANES lanes per particle; lane 0 writes the particle back.
+template <typename TF>
+__global__ __launch_bounds__(BEAM_THREADS) void k_beam_move(
+    BeamGeom g, int64_t n, double xi_k, double xi_k1, const double *__restrict__ q_m,
+    const double *__restrict__ dt, Fields6<TF> fk, Fields6<TF> fk1, int64_t *__restrict__ steps,
+    int64_t *__restrict__ id, double *__restrict__ x, double *__restrict__ y,
+    double *__restrict__ xi, double *__restrict__ px, double *__restrict__ py,
+    double *__restrict__ pz, uint8_t *__restrict__ lost, uint8_t *__restrict__ moved,
+    uint8_t *__restrict__ fell, unsigned *err)
+{
+    const int64_t t = blockIdx.x * (int64_t)BEAM_THREADS + threadIdx.x;
+    const int64_t k = t / BEAM_LANES;
+    const int lane = (int)(t % BEAM_LANES);
+    if (k >= n) return;   // whole groups: n particles fill BEAM_LANES n lanes
+    BeamState b{x[k], y[k], xi[k], px[k], py[k], pz[k], steps[k], false, false, false};
+    move_particle<TF>(g, xi_k, xi_k1, q_m[k], dt[k], fk, fk1, lane, b);
+    if (b.off) atomicOr(err, ERR_BEAM_OFF_GRID);
+    if (lane != 0) return;
+    if (b.lost) id[k] = -id[k];
+    x[k] = b.x;
+    y[k] = b.y;
+    xi[k] = b.xi;
+    px[k] = b.px;
+    py[k] = b.py;
+    pz[k] = b.pz;
+    steps[k] = b.steps;
+    lost[k] = b.lost;
+    fell[k] = b.fell;
+    moved[k] = !b.fell && !b.lost;
+}
+
+// ---- one layer's advance ---------------------------------------------------------------
+// lc3d_beam_advance: substep counts, move and split of a layer that is the
+// rows of two packed column ranges (the layout layer, then the particles that
+// fell into it), in two launches, where the separate calls copied both ranges
+// into one layer first and took three.  The rows are BeamRows' order.
+enum { BF_XI = 0, BF_X, BF_Y, BF_PX, BF_PY, BF_PZ, BF_QM, BF_QNORM, BF_DT, BEAM_F };
+enum { BI_ID = 0, BI_STEPS, BEAM_I };
+constexpr int BEAM_GROUPS = 3;                                  // lost, moved, fell
+constexpr int ADVANCE_PARTICLES = BEAM_THREADS / BEAM_LANES;    // of a block
+static_assert(ADVANCE_PARTICLES == 32, "BeamScratch");
+
+// Moves the particles into sc.f / sc.i (packed rows of n), their groups as
+// bits into sc.group and each block's group sizes into sc.count.
+template <typename TF>
+__global__ __launch_bounds__(BEAM_THREADS) void k_beam_advance(BeamGeom g, BeamRows layer,
+                                                               BeamRows fell, double xi_k,
+                                                               double xi_k1, double e_sub,
+                                                               double time_step, Fields6<TF> fk,
+                                                               Fields6<TF> fk1, BeamScratch sc,
+                                                               unsigned *err)
+{
+    __shared__ int s_count[BEAM_THREADS / 64][BEAM_GROUPS];
+    const int64_t n = layer.n + fell.n;
+    const int64_t t = blockIdx.x * (int64_t)BEAM_THREADS + threadIdx.x;
+    const int64_t k = t / BEAM_LANES;
+    const int lane = (int)(t % BEAM_LANES);
+    unsigned group = 0;
+    if (k < n) {   // whole groups
+        const bool laid = k < layer.n;
+        const BeamRows &from = laid ? layer : fell;
+        const int64_t c = laid ? k : k - layer.n;
+        const double *f = from.f + c;
+        const int64_t fs = from.f_stride;
+        const int64_t *iv = from.i + c;
+        const double qm = f[BF_QM * fs];
+        double dt = f[BF_DT * fs];
+        BeamState b{f[BF_X * fs],  f[BF_Y * fs],  f[BF_XI * fs],
+                    f[BF_PX * fs], f[BF_PY * fs], f[BF_PZ * fs],
+                    iv[BI_STEPS * from.i_stride], false, false, false};
+        if (laid) substeps_of(qm, b.pz, e_sub, time_step, dt, b.steps);
+        move_particle<TF>(g, xi_k, xi_k1, qm, dt, fk, fk1, lane, b);
+        if (b.off) atomicOr(err, ERR_BEAM_OFF_GRID);
+        if (lane == 0) {
+            group = (b.lost ? 1u : 0u) | (!b.fell && !b.lost ? 2u : 0u) | (b.fell ? 4u : 0u);
+            const int64_t id = iv[BI_ID * from.i_stride];
+            double *o = sc.f + k;
+            o[BF_XI * n] = b.xi;
+            o[BF_X * n] = b.x;
+            o[BF_Y * n] = b.y;
+            o[BF_PX * n] = b.px;
+            o[BF_PY * n] = b.py;
+            o[BF_PZ * n] = b.pz;
+            o[BF_QM * n] = qm;
+            o[BF_QNORM * n] = f[BF_QNORM * fs];
+            o[BF_DT * n] = dt;
+            sc.i[BI_ID * n + k] = b.lost ? -id : id;
+            sc.i[BI_STEPS * n + k] = b.steps;
+            sc.group[k] = (uint8_t)group;
+        }
+    }
+    const int wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < BEAM_GROUPS; ++q) {
+        const int c = __builtin_popcountll(__ballot((group >> q) & 1u));
+        if ((threadIdx.x & 63) == 0) s_count[wave][q] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x < BEAM_GROUPS) {
+        int c = 0;
+        for (int w = 0; w < BEAM_THREADS / 64; ++w) c += s_count[w][threadIdx.x];
+        sc.count[threadIdx.x * (int64_t)gridDim.x + blockIdx.x] = c;
+    }
+}
+
+// Group q's particles to the front of out_f + q BEAM_F n and out_i + q BEAM_I n,
+// in layer order: a block's particles go behind those that the blocks of
+// k_beam_advance before it counted.
+constexpr int PLACE_THREADS = 256;
+__global__ __launch_bounds__(PLACE_THREADS) void k_beam_place(int64_t n, int blocks, BeamScratch sc,
+                                                              double *__restrict__ out_f,
+                                                              int64_t *__restrict__ out_i,
+                                                              int64_t *__restrict__ counts)
+{
+    constexpr int WAVES = PLACE_THREADS / 64, PER = PLACE_THREADS / ADVANCE_PARTICLES;
+    __shared__ int s_before[WAVES][BEAM_GROUPS], s_wave[WAVES][BEAM_GROUPS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t k = blockIdx.x * (int64_t)PLACE_THREADS + threadIdx.x;
+    const unsigned group = k < n ? sc.group[k] : 0u;
+    unsigned long long in[BEAM_GROUPS];
+#pragma unroll
+    for (int q = 0; q < BEAM_GROUPS; ++q) {
+        in[q] = __ballot((group >> q) & 1u);
+        const int mine = (int)blockIdx.x * PER;
+        int c = 0;
+        for (int b = threadIdx.x; b < mine; b += PLACE_THREADS) c += sc.count[q * (int64_t)blocks + b];
+        // Exact in double: at most 2^31 particles.
+        double v = (double)c;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+        if (lane == 0) {
+            s_before[wave][q] = (int)v;
+            s_wave[wave][q] = __builtin_popcountll(in[q]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < BEAM_GROUPS; ++q) {
+        int64_t at = 0, total = 0;
+        for (int w = 0; w < WAVES; ++w) {
+            at += s_before[w][q] + (w < wave ? s_wave[w][q] : 0);
+            total += s_before[w][q] + s_wave[w][q];
+        }
+        if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) counts[q] = total;
+        if ((group >> q) & 1u) {
+            at += __builtin_popcountll(in[q] & ((1ull << lane) - 1ull));
+            double *of = out_f + q * (int64_t)BEAM_F * n + at;
+            int64_t *oi = out_i + q * (int64_t)BEAM_I * n + at;
+            double v[BEAM_F];
+            int64_t w[BEAM_I];
+#pragma unroll
+            for (int r = 0; r < BEAM_F; ++r) v[r] = sc.f[r * n + k];
+#pragma unroll
+            for (int r = 0; r < BEAM_I; ++r) w[r] = sc.i[r * n + k];
+#pragma unroll
+            for (int r = 0; r < BEAM_F; ++r) of[r * n] = v[r];
+#pragma unroll
+            for (int r = 0; r < BEAM_I; ++r) oi[r * n] = w[r];
+        }
+    }
 }
 
 // beam_calculator.py:124-139 (the split of a moved layer): for each group g
@@ -385,6 +546,24 @@ hipError_t launch_beam_split(int64_t n, int nf, int ni, const double *f, const i
     const unsigned bx = chunks >= 2 && chunks <= SPLIT_MAX_BLOCKS ? (unsigned)chunks : 1u;
     k_beam_split<<<dim3(bx, 3), SPLIT_THREADS, 0, s>>>(n, nf, ni, f, iv, flags, out_f, out_i,
                                                         counts);
+    return hipGetLastError();
+}
+
+hipError_t launch_beam_advance(const BeamGeom &g, const BeamRows &layer, const BeamRows &fell,
+                               int64_t beam_layer_idx, double e_sub, double time_step,
+                               const Fields6<double> &fk, const Fields6<double> &fk1,
+                               const BeamScratch &sc, double *out_f, int64_t *out_i,
+                               int64_t *counts, unsigned *err, hipStream_t s)
+{
+    const int64_t n = layer.n + fell.n;
+    if (n <= 0) return hipSuccess;
+    const double xi_k = (double)beam_layer_idx * -g.xi_step;
+    const double xi_k1 = (double)(beam_layer_idx + 1) * -g.xi_step;
+    const int blocks = (int)((n + ADVANCE_PARTICLES - 1) / ADVANCE_PARTICLES);
+    k_beam_advance<double><<<blocks, BEAM_THREADS, 0, s>>>(g, layer, fell, xi_k, xi_k1, e_sub,
+                                                           time_step, fk, fk1, sc, err);
+    k_beam_place<<<(unsigned)((n + PLACE_THREADS - 1) / PLACE_THREADS), PLACE_THREADS, 0, s>>>(
+        n, blocks, sc, out_f, out_i, counts);
     return hipGetLastError();
 }
 

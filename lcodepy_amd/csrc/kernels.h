@@ -319,6 +319,34 @@ hipError_t launch_beam_move(const BeamGeom &g, int64_t n, int64_t beam_layer_idx
                             uint8_t *lost, uint8_t *moved, uint8_t *fell, unsigned *err,
                             hipStream_t s);
 
+// A range of n columns of packed beam rows: float64 row r of column c (xi x y
+// px py pz q_m q_norm dt) at f[r f_stride + c], int64 row r (id, remaining
+// steps) at i[r i_stride + c].
+struct BeamRows {
+    int64_t n;
+    const double *f;
+    int64_t f_stride;
+    const int64_t *i;
+    int64_t i_stride;
+};
+
+// Scratch of launch_beam_advance for n particles: the moved rows (packed, 9 n
+// and 2 n), group sizes per 32 particles (3 ceil(n / 32)), group bits (n).
+struct BeamScratch {
+    double *f;
+    int64_t *i;
+    int *count;
+    uint8_t *group;
+};
+
+// Substeps (of the layer's particles; the fallen ones keep theirs), move and
+// order-preserving split of the layer followed by the fallen particles.
+hipError_t launch_beam_advance(const BeamGeom &g, const BeamRows &layer, const BeamRows &fell,
+                               int64_t beam_layer_idx, double e_sub, double time_step,
+                               const Fields6<double> &fk, const Fields6<double> &fk1,
+                               const BeamScratch &sc, double *out_f, int64_t *out_i,
+                               int64_t *counts, unsigned *err, hipStream_t s);
+
 // Order-preserving split of a moved layer's nf float64 and ni int64 rows (n
 // particles each) by the three flag rows (lost, moved, fell): group g's
 // particles to the front of out_f[g] (nf x n) and out_i[g] (ni x n), their

@@ -6,8 +6,6 @@ three pushes, three deposits and two field solves as one stream-ordered
 sequence of HIP kernels (lc3d_plasma_step), with no host round trip."""
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from .. import _native, runtime
@@ -15,7 +13,7 @@ from .._native import ptr, stream_ptr
 from ..config import Config
 from . import _bind
 from .data import Arrays
-from .fields import get_field_computer, new_fields
+from .fields import FIELD_KEYS, get_field_computer, new_fields
 from .move import get_plasma_particles_mover
 from .rhoj import get_rhoj_computer
 
@@ -46,7 +44,7 @@ class Plane2d3vPlasmaSolver:
         structs = (_native.Sort * len(sorts))()
         for i, (sort, column) in enumerate(sorts):
             prev = particles_prev[sort]
-            _bind.check_sort(prev, dt)
+            x_init, y_init, x_offt, y_offt, px, py, pz, q, m = _bind.checked_pointers(prev, dt)
             full = Arrays.wrap(
                 x_init=prev.x_init, y_init=prev.y_init, m=prev.m,
                 x_offt=torch.empty_like(prev.x_offt), y_offt=torch.empty_like(prev.y_offt),
@@ -55,7 +53,11 @@ class Plane2d3vPlasmaSolver:
                 **{k: getattr(prev, k) for k in prev.names()
                    if k not in _bind.PARTICLE_KEYS})
             particles_full[sort] = full
-            structs[i] = _bind.sort_struct(prev, full, column)
+            # The arrays of layer k+1 are fresh, and m is the same tensor.
+            structs[i] = _native.Sort(
+                prev.m.numel(), x_init, y_init, m, x_offt, y_offt, px, py, q, pz,
+                full.x_offt.data_ptr(), full.y_offt.data_ptr(), full.px.data_ptr(),
+                full.py.data_ptr(), full.q.data_ptr(), full.pz.data_ptr(), column)
             if self.declustering_enabled and i == 0:
                 z = lambda: torch.zeros_like(prev.x_offt, dtype=torch.float64)
                 dxp = getattr(prev, 'dx_chaotic', None)
@@ -67,7 +69,11 @@ class Plane2d3vPlasmaSolver:
                 s.dx_chaotic_prev, s.dy_chaotic_prev = dxp.data_ptr(), dyp.data_ptr()
                 s.dx_chaotic, s.dy_chaotic = full.dx_chaotic.data_ptr(), full.dy_chaotic.data_ptr()
         fields_full = new_fields(N, dt.full)
-        fields_half = new_fields(N, dt.half)
+        # The half-step fields are the step's own: seven grids of one tensor.
+        half = torch.empty(7, N, N, dtype=dt.half, device=dev)
+        grid_bytes = half.stride(0) * half.element_size()
+        fields_half = _native.Fields(*range(half.data_ptr(), half.data_ptr() + 7 * grid_bytes,
+                                            grid_bytes))
         cur = Arrays.wrap(**{k: torch.empty(2, N, N, dtype=dt.current, device=dev)
                              for k in ('ro', 'jx', 'jy', 'jz')})
         bg = None
@@ -82,8 +88,10 @@ class Plane2d3vPlasmaSolver:
         rbf = rho_beam_full.to(dt.beam_rho).contiguous()
         rbp = rho_beam_prev.to(dt.beam_rho).contiguous()
         self.ctx.check(self.ctx.lib.lc3d_plasma_step(
-            self.ctx.handle, len(sorts), structs, ctypes.byref(_bind.fields7(fields_prev)),
-            ctypes.byref(_bind.currents(currents_prev)), ptr(rbf), ptr(rbp), ptr(bg),
-            ctypes.byref(_bind.fields7(fields_full)), ctypes.byref(_bind.fields7(fields_half)),
-            ctypes.byref(_bind.currents(cur)), stream_ptr()), 'lc3d_plasma_step')
+            self.ctx.handle, len(sorts), structs, _bind.fields7(fields_prev),
+            _bind.currents(currents_prev), ptr(rbf), ptr(rbp), ptr(bg),
+            _native.Fields(*[getattr(fields_full, k).data_ptr() for k in FIELD_KEYS]),
+            fields_half, _native.Currents(cur.ro.data_ptr(), cur.jx.data_ptr(),
+                                          cur.jy.data_ptr(), cur.jz.data_ptr()),
+            stream_ptr()), 'lc3d_plasma_step')
         return particles_full, fields_full, cur

@@ -1,7 +1,7 @@
 """The xi loop of one time step (push_solvers/push_solver.py:189-286)."""
 from __future__ import annotations
 
-from .beam3d.beam_calculator import BeamCalculator, RigidBeamCalculator
+from .beam3d.beam_calculator import BeamCalculator, PendingMove, RigidBeamCalculator
 from .beam3d.data import BeamParticles
 from .config import Config
 from .plasma3d.solver import Plane2d3vPlasmaSolver
@@ -71,7 +71,7 @@ class PusherAndSolver3D:
         side = None if rigid else torch.cuda.Stream(device=runtime.device())
         ro_beam_prev = torch.zeros(N, N, dtype=torch.float64, device=runtime.device())
         self.ez_axis = []
-        pending, prev_layout, fell_size = None, None, 0
+        pending, prev_layout = None, None
         start = round(-xi_plasma_layer_start / self.xi_step_size) + 1
 
         on_side = [False]   # whether the last deposit ran on the beam stream
@@ -104,7 +104,9 @@ class PusherAndSolver3D:
                 ro_beam_full = self.beam_calculator.layout_beam_layer(beam_layer_to_layout, xi_i)
             else:
                 beam_layer_to_layout, ro_beam_full, ready = next_layout
-                if ready is not None:
+                # A deposit that has ended needs no wait (which would cost
+                # the host more than everything else of the layer).
+                if ready is not None and not ready.query():
                     main.wait_event(ready)
             prev_plasma_fields = plasma_fields   # step_dxi returns fresh objects
             plasma_particles, plasma_fields, plasma_currents = self.plasma_solver.step_dxi(
@@ -112,13 +114,11 @@ class PusherAndSolver3D:
                 ro_beam_full, ro_beam_prev)
             if not rigid:
                 next_layout = layout_ahead(xi_i + 1) if xi_i < self.xi_steps else None
-                beam_layer_to_move = self.beam_particles_class()
                 fell = None
                 if pending is not None:
                     _lost, moved, fell = pending.result()
                     _read_on(moved, main)
                     beam_drain.push_beam_layer(moved)
-                    fell_size = fell.size
                 if fell is not None and prev_layout.size + fell.size > 0:
                     fields_ready = torch.cuda.Event()
                     fields_ready.record(main)
@@ -129,14 +129,10 @@ class PusherAndSolver3D:
                             if isinstance(t, torch.Tensor):
                                 t.record_stream(side)
                     with torch.cuda.stream(side):
-                        beam_layer_to_move.append(prev_layout).append(fell)
-                        pending = self.beam_calculator.move_beam_layer_async(
-                            beam_layer_to_move, fell_size, xi_i, prev_plasma_fields,
-                            plasma_fields)
+                        pending = self.beam_calculator.advance_layer_async(
+                            prev_layout, fell, xi_i, prev_plasma_fields, plasma_fields)
                 else:
-                    # nothing to move: no kernel is launched
-                    pending = self.beam_calculator.move_beam_layer_async(
-                        beam_layer_to_move, fell_size, xi_i, prev_plasma_fields, plasma_fields)
+                    pending = PendingMove(None, None, None, None)   # nothing to move
                 prev_layout = beam_layer_to_layout
             # The beam calculator hands over a fresh density each step; a rigid
             # beam's callable may return its own buffer.

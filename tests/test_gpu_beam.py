@@ -129,6 +129,42 @@ def test_beam_move_substeps_losses_and_falls_match_oracle():
         assert np.array_equal(g.remaining_steps.cpu().numpy(), o['remaining_steps']), name
 
 
+@pytest.mark.parametrize('n_layer,n_fell', [(0, 5), (1, 0), (31, 1), (32, 0), (255, 2), (256, 300),
+                                           (5000, 700)])
+def test_beam_advance_equals_the_separate_calls(n_layer, n_fell):
+    """lc3d_beam_advance of a layer and the particles fallen into it, both
+    column slices of wider packed rows, against substep, move and split of the
+    joined layer, bit for bit (each particle's arithmetic is the same): one
+    particle, both sides of the 32 particles of a moving block and of the 256
+    of a placing one, a block that holds both ranges, and many."""
+    from lcodepy_amd.beam3d.beam_calculator import BeamCalculator
+    from lcodepy_amd.beam3d.data import FLOAT_KEYS, INT_KEYS, BeamParticles
+    from lcodepy_amd.plasma3d.data import Arrays
+    print(f'beam advance {n_layer} + {n_fell}', flush=True)
+    rng = np.random.default_rng(n_layer + 7 * n_fell)
+    b = _layer(rng)
+    pick = rng.integers(0, b['x'].size, n_layer + n_fell + 9)
+    f = torch.tensor(np.stack([b[k] for k in FLOAT_KEYS])[:, pick], device='cuda')
+    i = torch.tensor(np.stack([b[k] for k in INT_KEYS])[:, pick], device='cuda')
+    f[8] = TIME_STEP / 2                                # dt and steps of the fallen
+    i[1] = torch.arange(i.shape[1], device='cuda') % 3
+    i[0] = torch.arange(1, i.shape[1] + 1, device='cuda')
+    rows = BeamParticles(f=f, i=i)
+    layer, fell = rows.slice(4, 4 + n_layer), rows.slice(4 + n_layer, 4 + n_layer + n_fell)
+    fields = [Arrays.wrap(**{k: torch.tensor(_smooth(rng, 0.05), device='cuda')
+                             for k in ('Ex', 'Ey', 'Ez', 'Bx', 'By', 'Bz')}) for _ in range(2)]
+    calc = BeamCalculator(_config())
+    before = rows.f.clone(), rows.i.clone()
+    got = calc.advance_layer_async(layer, fell, LAYER, *fields).result()
+    assert torch.equal(rows.f, before[0]) and torch.equal(rows.i, before[1])
+    joined = BeamParticles().append(rows.slice(4, 4 + n_layer + n_fell))
+    want = calc.move_beam_layer(joined, n_fell, LAYER, *fields)
+    calc.ctx.raise_on_errors()
+    assert sum(g.size for g in got) >= n_layer + n_fell
+    for g, w in zip(got, want):
+        assert torch.equal(g.f, w.f) and torch.equal(g.i, w.i)
+
+
 @pytest.mark.parametrize('n', [1, 700, 1024, 5000, 32 * 1024, 40000])
 def test_beam_split_keeps_layer_order(n):
     """lc3d_beam_split (beam_calculator.py:124-139) against numpy's boolean
