@@ -542,7 +542,7 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
               hipMalloc(&c->pid, cap * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->pos, cap * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->big, dense_cell_capacity(cap) * sizeof(int)) == hipSuccess &&
-              hipMalloc(&c->nbig, sizeof(int)) == hipSuccess &&
+              hipMalloc(&c->nbig, 2 * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->dslot, nkeys * sizeof(int)) == hipSuccess &&
               hipMalloc(&c->dense, dense_cell_capacity(cap) * 100 * tg) == hipSuccess &&
               hipMalloc(&c->work, 7 * nn * tg) == hipSuccess &&
@@ -619,7 +619,7 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
     if (e == hipSuccess) e = hipMemset(c->count, 0, (nkeys + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->base, 0, c->nbase * sizeof(int));
-    if (e == hipSuccess) e = hipMemset(c->nbig, 0, sizeof(int));
+    if (e == hipSuccess) e = hipMemset(c->nbig, 0, 2 * sizeof(int));
     c->bigcap = dense_cell_capacity(cap);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {

@@ -123,7 +123,7 @@ __device__ __forceinline__ void clear_scan(const BinState &bs)
 {
     if (blockIdx.x != 0) return;
     for (int i = threadIdx.x; i < bs.nbase; i += blockDim.x) bs.base[i] = 0;
-    if (threadIdx.x == 0) *bs.nbig = 0;
+    if (threadIdx.x < 2) bs.nbig[threadIdx.x] = 0;
 }
 
 // Counts the particles of a wave into their cells and returns each one's

@@ -42,6 +42,7 @@ constexpr int SCAN_PER = 8;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_PER;
 static_assert(SCAN_TILE == SCAN_TILE_CELLS, "scan tiles as allocated");
 constexpr int SMALL_CELL = 16;          // lists a gather thread sorts; longer ones are dense
+constexpr int WAVE_CELL = 64;           // dense lists up to this long are one wave's
 constexpr int MAX_SORTED_CELL = 16384;  // lists sorted by a workgroup in LDS
 
 // ---- binning ------------------------------------------------------------------
@@ -117,7 +118,8 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *sh, int &total)
 // lstart[c] + base[c / SCAN_TILE] (list_start).  base and the queue of dense
 // cells are empty when the pass begins (the binning pass clears them); a dense
 // cell takes a slot of the queue (at most n / (SMALL_CELL + 1) < bigcap cells
-// can be dense), and dslot is written, and read, for dense cells only.
+// can be dense), those of at most WAVE_CELL particles from its front and the
+// others from its back, and dslot is written, and read, for dense cells only.
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_cells(int ncell, int ntiles, BinState bs)
 {
     __shared__ int sh[SCAN_THREADS / 64];
@@ -138,8 +140,11 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_cells(int ncell, int ntil
         if (first + i < ncell) count[first + i] = 0;
         run += c[i];
         if (c[i] > SMALL_CELL) {
-            const int slot = atomicAdd(bs.nbig, 1);
-            if (slot < bs.bigcap) bs.big[slot] = first + i;
+            // Two atomics, so that each is at one address and a wave's add as one.
+            int slot;
+            if (c[i] <= WAVE_CELL) slot = atomicAdd(&bs.nbig[0], 1);
+            else slot = bs.bigcap - 1 - atomicAdd(&bs.nbig[1], 1);
+            if (slot >= 0 && slot < bs.bigcap) bs.big[slot] = first + i;
             bs.dslot[first + i] = slot;
             if (c[i] > MAX_SORTED_CELL) atomicOr(bs.err, ERR_CELL_OVERFLOW);
         }
@@ -172,100 +177,234 @@ __global__ __launch_bounds__(256) void k_scatter(int64_t n, int ncell, BinState 
 }
 
 // ---- dense cells: sort and taps ------------------------------------------------------
-// One workgroup per dense cell, the grid striding over the queue.  The cell's
-// list is sorted by particle id with a bitonic sort of (particle id,
-// position) keys in LDS (lists of up to MAX_SORTED_CELL; longer ones keep
-// arrival order).  Then thread t sums its contiguous segment of the sorted list into the 5 x 5 taps x 4 currents
-// around the cell; the 256 partial sums are combined by a butterfly within
-// each wave and then the four waves in a fixed order.  out[slot][tap][q],
-// tap = 5 a + b for the target cell (ix + a - 2, iy + b - 2), q = ro jx jy jz.
+// The 5 x 5 taps x 4 currents around each dense cell, out[slot][tap][q], tap =
+// 5 a + b for the target cell (ix + a - 2, iy + b - 2), q = ro jx jy jz.  The
+// cell's list is sorted by particle id (lists of more than MAX_SORTED_CELL keep
+// arrival order); particle i of it is summed by thread i (of DENSE_THREADS,
+// each a contiguous segment of a longer list), and the threads' sums are
+// combined by a butterfly within each wave and then the four waves in a fixed
+// order.  The butterfly hands half of the values that are left to the partner
+// lane at every step (a sixth of the shuffles, the same sums).
+//
+// A list of at most WAVE_CELL particles is one wave's, one of at most
+// DENSE_THREADS four waves', which rank it by comparing ids; a longer one is
+// sorted in the workgroup's LDS.  One workgroup per list of any length left 4
+// waves on a CU (N = 513, 16 ppc, float64: 2424 -> 144 us; lists of about 180,
+// N = 417, float32: 30 -> 25 us).
 constexpr int DENSE_VALUES = 25 * 4;
-constexpr int DENSE_THREADS = 256;
+constexpr int DENSE_THREADS = 256;   // of a list longer than a wave
+constexpr int DENSE_BLOCK = 2 * DENSE_THREADS, DENSE_WAVES = DENSE_BLOCK / 64;
+
+// Two of the four currents of one particle at a time (PAIR_VALUES sums a
+// lane: all four would spill in float64): acc[2 (5 a + b) + r] += c_r w_a w_b.
+constexpr int PAIR_VALUES = DENSE_VALUES / 2;
 template <typename T>
-__global__ __launch_bounds__(DENSE_THREADS) void k_dense_cells(double h, BinState bs)
+__device__ __forceinline__ void add_pair_taps(const DepRec<T> &d, int pair, T inv_h,
+                                              T (&acc)[PAIR_VALUES])
+{
+    const T c0 = pair ? d.c2 : d.c0, c1 = pair ? d.c3 : d.c1;
+    T wx[5], wy[5];
+    weights4<T>(d.xl, wx);
+    weights4<T>(d.yl, wy);
+#pragma unroll
+    for (int a = 0; a < 5; ++a) {
+#pragma unroll
+        for (int b = 0; b < 5; ++b) {
+            const T w = (wx[a] * inv_h) * (wy[b] * inv_h);
+            acc[2 * (5 * a + b) + 0] += c0 * w;
+            acc[2 * (5 * a + b) + 1] += c1 * w;
+        }
+    }
+}
+
+// One step of the halving butterfly: M values at distance off become (M + 1) / 2,
+// the sums over the lane pair of the lower half (lanes without bit off) or
+// the upper one.
+template <int M, typename T, int K>
+__device__ __forceinline__ void halve(T (&v)[K], int off, bool upper)
+{
+    constexpr int H = (M + 1) / 2;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        const T lo = v[k], hi = H + k < M ? v[H + k] : T(0);
+        v[k] = (upper ? hi : lo) + __shfl_xor(upper ? lo : hi, off);
+    }
+}
+
+// The sums of a wave's PAIR_VALUES: lane's is value wave_value(lane), or none (-1).
+template <typename T>
+__device__ __forceinline__ T wave_sums(T (&v)[PAIR_VALUES], int lane)
+{
+    halve<50>(v, 32, lane & 32);
+    halve<25>(v, 16, lane & 16);
+    halve<13>(v, 8, lane & 8);
+    halve<7>(v, 4, lane & 4);
+    halve<4>(v, 2, lane & 2);
+    halve<2>(v, 1, lane & 1);
+    return v[0];
+}
+__device__ __forceinline__ int wave_value(int lane)
+{
+    constexpr int KEPT[6] = {25, 13, 7, 4, 2, 1};   // by the lower half of each step
+    int value = 0, left = PAIR_VALUES;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const bool upper = lane & (32 >> k);
+        value += upper ? KEPT[k] : 0;
+        left = upper ? left - KEPT[k] : min(left, KEPT[k]);
+    }
+    return left > 0 ? value : -1;
+}
+
+template <typename T>
+__global__ __launch_bounds__(DENSE_BLOCK) void k_dense_cells(double h, BinState bs)
 {
     __shared__ unsigned long long s[MAX_SORTED_CELL];   // particle id << 32 | position
-    __shared__ T red[4][DENSE_VALUES];
-    const int nbig = min(*bs.nbig, bs.bigcap);
+    __shared__ T red[DENSE_WAVES][PAIR_VALUES];
+    const int few = min(bs.nbig[0], bs.bigcap), many = min(bs.nbig[1], bs.bigcap - few);
     const DepRec<T> *__restrict__ rec = static_cast<const DepRec<T> *>(bs.rec);
     T *__restrict__ out = static_cast<T *>(bs.dense);
     const int t = threadIdx.x, lane = t % 64, wave = t / 64;
     const T inv_h = T(1.0 / h);
-    for (int b = blockIdx.x; b < nbig; b += gridDim.x) {
+    const int value = wave_value(lane);
+
+    for (int b = blockIdx.x * DENSE_WAVES + wave; b < few; b += gridDim.x * DENSE_WAVES) {
         const int c = bs.big[b];
-        const int st = list_start(bs, c), n = list_start(bs, c + 1) - st;   // n > SMALL_CELL
-        const bool sorted = n <= MAX_SORTED_CELL;
-        if (sorted) {
-            int P = 1;
-            while (P < n) P <<= 1;
-            for (int i = t; i < P; i += DENSE_THREADS) {
-                unsigned long long v = ~0ull;
-                if (i < n)
-                    v = (unsigned long long)(unsigned)bs.idx[st + i] << 32 | (unsigned)bs.pos[st + i];
-                s[i] = v;
+        const int st = list_start(bs, c), n = list_start(bs, c + 1) - st;   // n <= WAVE_CELL
+        int id = INT_MAX, at = 0;
+        if (lane < n) {
+            id = bs.idx[st + lane];
+            at = bs.pos[st + lane];
+        }
+        // Lane i takes the particle whose id has i smaller ones before it.
+        int place = 0, from = 0;
+        for (int j = 0; j < n; ++j) place += __shfl(id, j) < id ? 1 : 0;
+        for (int j = 0; j < n; ++j)
+            if (__shfl(place, j) == lane) from = j;
+        at = __shfl(at, from);
+        DepRec<T> d{};
+        if (lane < n) d = rec[at];
+#pragma unroll 1
+        for (int pair = 0; pair < 2; ++pair) {
+            T acc[PAIR_VALUES];
+#pragma unroll
+            for (int k = 0; k < PAIR_VALUES; ++k) acc[k] = T(0);
+            if (lane < n) add_pair_taps<T>(d, pair, inv_h, acc);
+            const T v = wave_sums(acc, lane);
+            if (value >= 0)
+                out[(size_t)b * DENSE_VALUES + 4 * (value / 2) + 2 * pair + value % 2] = v;
+        }
+    }
+
+    // The longer lists, two to a workgroup: half of its waves each.  Every
+    // thread reaches the barriers, also without a list.
+    const int half = t / DENSE_THREADS, u = t % DENSE_THREADS;
+    int *ids = reinterpret_cast<int *>(s) + half * 2 * DENSE_THREADS, *order = ids + DENSE_THREADS;
+    for (int b0 = 2 * blockIdx.x; b0 < many; b0 += 2 * gridDim.x) {
+        {
+            const int b = bs.bigcap - 1 - (b0 + half);
+            int st = 0, n = 0;
+            if (b0 + half < many) {
+                const int c = bs.big[b];
+                st = list_start(bs, c);
+                n = list_start(bs, c + 1) - st;
+                if (n > DENSE_THREADS) n = 0;
             }
+            int id = INT_MAX, at = 0;
+            if (u < n) {
+                id = bs.idx[st + u];
+                at = bs.pos[st + u];
+            }
+            ids[u] = id;
             __syncthreads();
-            for (int k = 2; k <= P; k <<= 1) {
-                for (int j = k >> 1; j > 0; j >>= 1) {
-                    for (int i = t; i < P; i += DENSE_THREADS) {
-                        const int l = i ^ j;
-                        if (l > i) {
-                            const unsigned long long x = s[i], y = s[l];
-                            if ((x > y) == ((i & k) == 0)) {
-                                s[i] = y;
-                                s[l] = x;
+            int rank = 0;
+            for (int j = 0; j < n; j += 4) {   // past the list: INT_MAX, not less
+                const int4 o = *reinterpret_cast<const int4 *>(ids + j);
+                rank += (o.x < id) + (o.y < id) + (o.z < id) + (o.w < id);
+            }
+            if (u < n) order[rank] = at;
+            __syncthreads();
+            DepRec<T> d{};
+            if (u < n) d = rec[order[u]];
+#pragma unroll 1
+            for (int pair = 0; pair < 2; ++pair) {
+                T acc[PAIR_VALUES];
+#pragma unroll
+                for (int k = 0; k < PAIR_VALUES; ++k) acc[k] = T(0);
+                if (u < n) add_pair_taps<T>(d, pair, inv_h, acc);
+                const T v = wave_sums(acc, lane);
+                if (value >= 0) red[wave][value] = v;
+                __syncthreads();
+                if (n > 0 && u < PAIR_VALUES) {
+                    const T (*r)[PAIR_VALUES] = red + half * (DENSE_THREADS / 64);
+                    out[(size_t)b * DENSE_VALUES + 4 * (u / 2) + 2 * pair + u % 2] =
+                        (r[0][u] + r[1][u]) + (r[2][u] + r[3][u]);
+                }
+                __syncthreads();
+            }
+        }
+        for (int k = b0; k < min(b0 + 2, many); ++k) {   // the whole block
+            const int b = bs.bigcap - 1 - k, c = bs.big[b];
+            const int st = list_start(bs, c), n = list_start(bs, c + 1) - st;
+            if (n <= DENSE_THREADS) continue;
+            const bool sorted = n <= MAX_SORTED_CELL;
+            if (sorted) {
+                int P = 1;
+                while (P < n) P <<= 1;
+                for (int i = t; i < P; i += DENSE_BLOCK) {
+                    unsigned long long v = ~0ull;
+                    if (i < n)
+                        v = (unsigned long long)(unsigned)bs.idx[st + i] << 32 |
+                            (unsigned)bs.pos[st + i];
+                    s[i] = v;
+                }
+                __syncthreads();
+                for (int w = 2; w <= P; w <<= 1) {
+                    for (int j = w >> 1; j > 0; j >>= 1) {
+                        for (int i = t; i < P; i += DENSE_BLOCK) {
+                            const int l = i ^ j;
+                            if (l > i) {
+                                const unsigned long long x = s[i], y = s[l];
+                                if ((x > y) == ((i & w) == 0)) {
+                                    s[i] = y;
+                                    s[l] = x;
+                                }
                             }
                         }
+                        __syncthreads();
                     }
-                    __syncthreads();
                 }
             }
-        }
-        const int seg = (n + DENSE_THREADS - 1) / DENSE_THREADS;
-        const int j0 = min(n, t * seg), j1 = min(n, (t + 1) * seg);
-        T acc[DENSE_VALUES];
+            // Both halves sum the list, a pair of currents each.
+            T acc[PAIR_VALUES];
 #pragma unroll
-        for (int k = 0; k < DENSE_VALUES; ++k) acc[k] = T(0);
-        for (int j = j0; j < j1; ++j) {
-            const DepRec<T> d = rec[sorted ? (int)(unsigned)s[j] : bs.pos[st + j]];
-            T wx[5], wy[5];
-            weights4<T>(d.xl, wx);
-            weights4<T>(d.yl, wy);
-#pragma unroll
-            for (int a = 0; a < 5; ++a) {
-#pragma unroll
-                for (int bb = 0; bb < 5; ++bb) {
-                    const T w = (wx[a] * inv_h) * (wy[bb] * inv_h);
-                    acc[(5 * a + bb) * 4 + 0] += d.c0 * w;
-                    acc[(5 * a + bb) * 4 + 1] += d.c1 * w;
-                    acc[(5 * a + bb) * 4 + 2] += d.c2 * w;
-                    acc[(5 * a + bb) * 4 + 3] += d.c3 * w;
-                }
+            for (int q = 0; q < PAIR_VALUES; ++q) acc[q] = T(0);
+            const int seg = (n + DENSE_THREADS - 1) / DENSE_THREADS;
+            const int j0 = min(n, u * seg), j1 = min(n, (u + 1) * seg);
+            for (int j = j0; j < j1; ++j)
+                add_pair_taps<T>(rec[sorted ? (int)(unsigned)s[j] : bs.pos[st + j]], half, inv_h,
+                                 acc);
+            const T v = wave_sums(acc, lane);
+            if (value >= 0) red[wave][value] = v;
+            __syncthreads();
+            if (u < PAIR_VALUES) {
+                const T (*r)[PAIR_VALUES] = red + half * (DENSE_THREADS / 64);
+                out[(size_t)b * DENSE_VALUES + 4 * (u / 2) + 2 * half + u % 2] =
+                    (r[0][u] + r[1][u]) + (r[2][u] + r[3][u]);
             }
+            __syncthreads();   // s and red are written again
         }
-#pragma unroll
-        for (int k = 0; k < DENSE_VALUES; ++k) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off);
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int k = 0; k < DENSE_VALUES; ++k) red[wave][k] = acc[k];
-        }
-        __syncthreads();
-        if (t < DENSE_VALUES)
-            out[(size_t)b * DENSE_VALUES + t] = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-        __syncthreads();
     }
 }
 
 // ---- gather deposit -------------------------------------------------------------------
-// One block per tile of TX x GATHER_TY output cells, one thread per output
-// row ox of the tile and source column cy (GATHER_TY + 4 = 32 of them, half a
-// wave).  The thread adds the particles of the five source cells (ox - 2 ..
-// ox + 2, cy), each with its x weight towards row ox, into the five y taps of
-// the four currents, in registers; the taps meet at the end by shuffles along
-// the half wave, where output cell (ox, o) takes tap b of column o + 2 - b.
+// One block per tile of TX x GATHER_TY output cells; per output row ox of the
+// tile and source column cy (GATHER_TY + 4 = 32 of them, half a wave) G
+// threads, each for 4 / G of the currents.  A thread adds the particles of the
+// five source cells (ox - 2 .. ox + 2, cy), each with its x weight towards row
+// ox, into the five y taps of its currents, in registers; the taps meet at the
+// end by shuffles along the half wave, where output cell (ox, o) takes tap b of
+// column o + 2 - b.
 //
 // The records of the source cells are staged in LDS, as many whole source
 // rows at a time as GatherPlan::cap holds (a row's lists of at most
@@ -275,16 +414,20 @@ __global__ __launch_bounds__(DENSE_THREADS) void k_dense_cells(double h, BinStat
 // two thirds of the time; the taps of every x offset also passed through LDS
 // with a barrier each, and 80 KB a block left two blocks to a CU.
 // Measured with the list sort it replaces: N = 513, 4 ppc 92 -> 55 us in
-// float64 and 48 -> 37 us in float32; 769, 9 ppc, float64 508 -> 238 us; 321, 4
-// ppc, float64 48 -> 35 us.  It is bound by the vector units (the waves run as
+// float64 and 48 -> 34 us in float32; 769, 9 ppc, float64 508 -> 238 us; 321, 4
+// ppc, float64 48 -> 32 us.  It is bound by the vector units (the waves run as
 // long as their fullest cells) and by the blocks' chain of list, record and
 // sum.  Staging with a thread per particle instead of a thread per cell took
 // 65 us in float32 (its ranks are a serial chain of LDS reads).
-// Blocks of TX = 8 rows below which the blocks take 4, so that a CU still
-// holds several (measured: N = 321 float64, 492 such blocks, 41 us against 35;
-// 417 float32, 795, 54 against 44; 513, 1235, 37 against 43 and, float64, 55
-// against 55; 769, 2716, 238 against 260).
-constexpr int GATHER_FEW = 1024;
+// A grid of fewer blocks of TX = 8, G = 1 than GATHER_FEW takes TX = 4, G = 2:
+// a CU holds several blocks, and each has more waves for its chain.  The
+// second weights cost less than that until the vector units are full.
+// Measured against TX = 8, G = 1 (N = 513: 1235 such blocks, 54.8 us against
+// 56.5 in float64 and 37.2 against 34.3 in float32; 769, 2716, float64, 237
+// against 271; 1025, 4773, float32, 118 against 125) and against TX = 4, G = 1
+// (281, 4 ppc, float32, 20.1 us against 26.0; 321 float64 32.4 against 35.0;
+// 129 float64 9.4 against 11.6).
+template <typename T> constexpr int GATHER_FEW = sizeof(T) == 4 ? 2048 : 1024;
 constexpr int GATHER_TY = 28, GATHER_COLS = GATHER_TY + 4;
 static_assert(GATHER_COLS == 32, "a source row is half a wave");
 // cap: records staged at a time (31 KB: five blocks a CU).
@@ -315,35 +458,32 @@ __device__ __forceinline__ void order_list(const int *__restrict__ idx,
     }
 }
 
-// Adds one particle's taps toward x offset A (target cells (ix + A - 2, iy +
-// b - 2)): tp[b][q] += c_q (w_A(xl) / h) (w_b(yl) / h).  Float32 takes the
-// current times the x weight first, float64 the weight product first
-// (plasma3d/weights.py:58-67).
-template <int A, typename T>
-__device__ __forceinline__ void add_taps(const DepRec<T> &d, T inv_h, T (&tp)[5][4])
+// Adds Q of a particle's currents, from the first'th on, to its taps toward x
+// offset A (target cells (ix + A - 2, iy + b - 2)): tp[b][q] += c_q (w_A(xl) / h)
+// (w_b(yl) / h).  Float32 takes the current times the x weight first, float64
+// the weight product first (plasma3d/weights.py:58-67).
+template <int A, int Q, typename T>
+__device__ __forceinline__ void add_taps(const DepRec<T> &d, int first, T inv_h, T (&tp)[5][Q])
 {
+    const T *c = &d.c0 + first;
     T wy[5];
     weights4<T>(d.yl, wy);
 #pragma unroll
     for (int b = 0; b < 5; ++b) wy[b] *= inv_h;
     const T wx = w4_tap<A, T>(d.xl) * inv_h;
     if constexpr (std::is_same<T, float>::value) {
-        const T c0 = d.c0 * wx, c1 = d.c1 * wx, c2 = d.c2 * wx, c3 = d.c3 * wx;
 #pragma unroll
-        for (int b = 0; b < 5; ++b) {
-            tp[b][0] += c0 * wy[b];
-            tp[b][1] += c1 * wy[b];
-            tp[b][2] += c2 * wy[b];
-            tp[b][3] += c3 * wy[b];
+        for (int q = 0; q < Q; ++q) {
+            const T cw = c[q] * wx;
+#pragma unroll
+            for (int b = 0; b < 5; ++b) tp[b][q] += cw * wy[b];
         }
     } else {
 #pragma unroll
         for (int b = 0; b < 5; ++b) {
             const T w = wx * wy[b];
-            tp[b][0] += d.c0 * w;
-            tp[b][1] += d.c1 * w;
-            tp[b][2] += d.c2 * w;
-            tp[b][3] += d.c3 * w;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) tp[b][q] += c[q] * w;
         }
     }
 }
@@ -352,14 +492,14 @@ __device__ __forceinline__ void add_taps(const DepRec<T> &d, T inv_h, T (&tp)[5]
 // per source column the five source cells in order, each cell's particles in
 // the order of their ids (float32: a cell's sum in float32, then float64),
 // then the five columns in float64; written by one thread.
-template <typename TP, typename TG, int TX>
-__global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
+template <typename TP, typename TG, int TX, int G>
+__global__ __launch_bounds__(TX *GATHER_COLS *G) void k_deposit_gather(
     int N, double h, BinState bs, TG *__restrict__ ro, TG *__restrict__ jx, TG *__restrict__ jy,
     TG *__restrict__ jz, const TG *__restrict__ bg_ro, TG *__restrict__ ro1, TG *__restrict__ jx1,
     TG *__restrict__ jy1, TG *__restrict__ jz1)
 {
     using T = TP;   // arithmetic type of the taps
-    constexpr int THREADS = TX * GATHER_COLS, ROWS = TX + 4, CELLS = ROWS * GATHER_COLS;
+    constexpr int Q = 4 / G, THREADS = TX * GATHER_COLS * G, ROWS = TX + 4, CELLS = ROWS * GATHER_COLS;
     constexpr int CAP = GatherPlan<T>::cap, CHUNKS = CELLS / 64, WAVES = THREADS / 64;
     static_assert(CELLS % 64 == 0, "the prefix takes whole waves of cells");
     __shared__ DepRec<T> s_rec[CAP];
@@ -413,13 +553,13 @@ __global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
     if (t == 0) s_off[0] = 0;
     __syncthreads();
 
-    const int cy = t % GATHER_COLS, ox = t / GATHER_COLS;
+    const int cy = t % GATHER_COLS, ox = t / GATHER_COLS % TX, g = t / (GATHER_COLS * TX);
     const T inv_h = T(1.0 / h);
-    double sum[5][4];
+    double sum[5][Q];
 #pragma unroll
     for (int b = 0; b < 5; ++b)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) sum[b][q] = 0;
+        for (int q = 0; q < Q; ++q) sum[b][q] = 0;
 
     int r0 = 0;
     while (r0 < ROWS) {   // source rows r0 .. r1 - 1, the same for every thread
@@ -443,7 +583,14 @@ __global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
             else order_list<4>(idx, pos, n, s_pos + off);
         }
         __syncthreads();
-        for (int i = t; i < total; i += THREADS) s_rec[i] = rec[s_pos[i]];
+        // Two records in flight a thread (57 -> 50 us where a few cells hold most
+        // of the plasma; four: slower where the lists are even).
+        for (int i = t; i < total; i += 2 * THREADS) {
+            const int j = min(i + THREADS, total - 1);
+            const DepRec<T> a = rec[s_pos[i]], b = rec[s_pos[j]];
+            s_rec[i] = a;
+            if (i + THREADS < total) s_rec[j] = b;
+        }
         __syncthreads();
         // Source row r reaches output row ox by x offset A = ox + 4 - r.
         auto visit = [&](auto a_const) {
@@ -452,27 +599,29 @@ __global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
             if (r < r0 || r >= r1) return;
             const int c = GATHER_COLS * r + cy, slot = s_dense[c];
             if (slot >= 0) {
-                const T *v = dense + (size_t)slot * DENSE_VALUES + 4 * (5 * A);
+                const T *v = dense + (size_t)slot * DENSE_VALUES + 4 * (5 * A) + Q * g;
 #pragma unroll
                 for (int b = 0; b < 5; ++b)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sum[b][q] += (double)v[4 * b + q];
+                    for (int q = 0; q < Q; ++q) sum[b][q] += (double)v[4 * b + q];
                 return;
             }
             const int e = s_off[c + 1] - base;
             if constexpr (std::is_same<T, float>::value) {
-                T tp[5][4];
+                T tp[5][Q];
 #pragma unroll
                 for (int b = 0; b < 5; ++b)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) tp[b][q] = T(0);
-                for (int i = s_off[c] - base; i < e; ++i) add_taps<A, T>(s_rec[i], inv_h, tp);
+                    for (int q = 0; q < Q; ++q) tp[b][q] = T(0);
+                for (int i = s_off[c] - base; i < e; ++i)
+                    add_taps<A, Q, T>(s_rec[i], Q * g, inv_h, tp);
 #pragma unroll
                 for (int b = 0; b < 5; ++b)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sum[b][q] += (double)tp[b][q];
+                    for (int q = 0; q < Q; ++q) sum[b][q] += (double)tp[b][q];
             } else {
-                for (int i = s_off[c] - base; i < e; ++i) add_taps<A, T>(s_rec[i], inv_h, sum);
+                for (int i = s_off[c] - base; i < e; ++i)
+                    add_taps<A, Q, T>(s_rec[i], Q * g, inv_h, sum);
             }
         };
         visit(std::integral_constant<int, 4>{});
@@ -485,9 +634,9 @@ __global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
     }
 
     // Output column o = cy of the tile sums tap b of source column cy + 4 - b.
-    double out[4];
+    double out[Q];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < Q; ++q) {
         out[q] = 0;
 #pragma unroll
         for (int b = 0; b < 5; ++b) out[q] += b < 4 ? __shfl(sum[b][q], (lane + 4 - b) & 63) : sum[b][q];
@@ -495,15 +644,12 @@ __global__ __launch_bounds__(TX *GATHER_COLS) void k_deposit_gather(
     const int gx = X0 + ox, gy = Y0 + cy;
     if (cy < GATHER_TY && gx < N && gy < N) {
         const int o = gx * N + gy;
-        ro[o] = (TG)out[0];
-        jx[o] = (TG)out[1];
-        jy[o] = (TG)out[2];
-        jz[o] = (TG)out[3];
-        if (bg_ro != nullptr) {
-            ro1[o] = bg_ro[o];
-            jx1[o] = 0;
-            jy1[o] = 0;
-            jz1[o] = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int c = Q * g + q;
+            (c == 0 ? ro : c == 1 ? jx : c == 2 ? jy : jz)[o] = (TG)out[q];
+            if (bg_ro != nullptr)
+                (c == 0 ? ro1 : c == 1 ? jx1 : c == 2 ? jy1 : jz1)[o] = c == 0 ? bg_ro[o] : TG(0);
         }
     }
 }
@@ -533,7 +679,7 @@ hipError_t launch_deposit(const PushGeom &g, const SortArrays<TP> &a, bool use_f
         k_scan_cells<<<ntiles, SCAN_THREADS, 0, s>>>(ncell, ntiles, bs);
         k_scatter<<<pblocks, 256, 0, s>>>(g.n, ncell, bs);
         // One block per CU (a block takes 134 KB of LDS): the queue is striding.
-        k_dense_cells<TP><<<256, DENSE_THREADS, 0, s>>>(g.h, bs);
+        k_dense_cells<TP><<<256, DENSE_BLOCK, 0, s>>>(g.h, bs);
     } else {
         // Empty sort: every cell list is empty (the binning pass, which has no
         // particle, clears what the scan adds to).
@@ -543,11 +689,11 @@ hipError_t launch_deposit(const PushGeom &g, const SortArrays<TP> &a, bool use_f
     const int tpr = (N + GATHER_TY - 1) / GATHER_TY;
     // Tile rows rounded up to a multiple of the XCDs.
     const int tiles8 = ((N + 7) / 8 + 7) / 8 * 8 * tpr, tiles4 = ((N + 3) / 4 + 7) / 8 * 8 * tpr;
-    if (tiles8 < GATHER_FEW)
-        k_deposit_gather<TP, TG, 4><<<tiles4, 4 * GATHER_COLS, 0, s>>>(
+    if (tiles8 < GATHER_FEW<TP>)
+        k_deposit_gather<TP, TG, 4, 2><<<tiles4, 8 * GATHER_COLS, 0, s>>>(
             N, g.h, bs, ro, jx, jy, jz, bg_ro, ro1, jx1, jy1, jz1);
     else
-        k_deposit_gather<TP, TG, 8><<<tiles8, 8 * GATHER_COLS, 0, s>>>(
+        k_deposit_gather<TP, TG, 8, 1><<<tiles8, 8 * GATHER_COLS, 0, s>>>(
             N, g.h, bs, ro, jx, jy, jz, bg_ro, ro1, jx1, jy1, jz1);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (timer) return timer->end(s);

@@ -63,8 +63,8 @@ struct BinState {
     unsigned *err;    // sticky error bits
     void *rec;        // per position: deposit records (deposit.hip)
     int64_t cap;      // particles the per-particle arrays hold
-    int *big;         // dense cells (more than 16 particles), in queue order
-    int *nbig;        // how many cells `big` holds
+    int *big;         // dense cells: of 17 to 64 particles from its front, more from its back
+    int *nbig;        // how many cells `big` holds from its front and its back
     int bigcap;       // capacity of `big`
     int *dslot;       // cell_keys(N): a dense cell's slot in `big`
     void *dense;      // per dense cell: its 5 x 5 x 4 deposit (deposit.hip)

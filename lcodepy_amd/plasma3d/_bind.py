@@ -5,20 +5,16 @@ from .. import _native
 from .._native import ptr
 
 PARTICLE_KEYS = ('x_init', 'y_init', 'x_offt', 'y_offt', 'px', 'py', 'pz', 'q', 'm')
-
-
-def _want(dt) -> tuple:
-    """(array, dtype) of a sort's arrays, in PARTICLE_KEYS' order."""
-    return tuple((k, dt.position if k in ('x_init', 'y_init', 'x_offt', 'y_offt')
-                  else dt.pz if k == 'pz' else dt.bulk) for k in PARTICLE_KEYS)
+POSITION_KEYS = ('x_init', 'y_init', 'x_offt', 'y_offt')
 
 
 def checked_pointers(a, dt) -> list:
     """Device addresses of the sort's arrays in PARTICLE_KEYS' order, each of
     them checked to be what the kernels take."""
     out = []
-    for k, want in _want(dt):
+    for k in PARTICLE_KEYS:
         t = getattr(a, k)
+        want = dt.position if k in POSITION_KEYS else dt.pz if k == 'pz' else dt.bulk
         if t.dtype != want or not t.is_cuda or not t.is_contiguous():
             raise TypeError(f'particle array {k}: need a contiguous {want} device tensor, '
                             f'got {t.dtype} on {t.device}')
@@ -27,7 +23,12 @@ def checked_pointers(a, dt) -> list:
 
 
 def check_sort(a, dt) -> None:
-    checked_pointers(a, dt)
+    for k in PARTICLE_KEYS:
+        t = getattr(a, k)
+        want = dt.position if k in POSITION_KEYS else dt.pz if k == 'pz' else dt.bulk
+        if t.dtype != want or not t.is_cuda or not t.is_contiguous():
+            raise TypeError(f'particle array {k}: need a contiguous {want} device tensor, '
+                            f'got {t.dtype} on {t.device}')
 
 
 def sort_struct(prev, full, column: int) -> _native.Sort:
