@@ -69,6 +69,36 @@ def test_noise_filter_matches_oracle(precision, damping):
         assert kick['px'] < 1e-10 and kick['py'] < 1e-10
 
 
+@pytest.mark.parametrize('N,averaging', [(33, 1), (45, 2), (65, 4), (97, 40)])
+def test_noise_filter_of_few_and_of_all_taps(N, averaging):
+    """Smoothing by taps over the whole period (averaging 1, 2 and 40) and by a
+    few of it, lattice sides on both sides of the outputs a thread sums.  Both
+    directions sum at most some hundred products with taps whose magnitudes sum
+    to less than 3, of about 1e-16 each: 1e-12 of the maximum."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.noise_filter import get_noise_filter
+    print(f'noise filter N={N} averaging {averaging}', flush=True)
+    cfg = _decl_cfg(N, 'fp64', 0.6)
+    cfg.set('declustering-averaging', averaging)
+    p = _params(N)
+    p.declustering = O.Declustering(averaging=averaging, force=0.3, damping=0.6, limit=1e-3)
+    el = O.uniform_plasma(p)
+    n = el['x_offt'].shape[0]
+    rng = np.random.default_rng(N)
+    for k in ('x_offt', 'y_offt'):
+        el[k] = 3e-4 * rng.standard_normal((n, n))
+    for k in ('px', 'py', 'pz'):
+        el[k] = 1e-3 * rng.standard_normal((n, n))
+    prev = {k: 1e-4 * rng.standard_normal((n, n)) for k in ('dx_chaotic', 'dy_chaotic')}
+    ref = O.noise_filter(p, {k: v.copy() for k, v in el.items()}, prev)
+    out = get_noise_filter(cfg)(Arrays.wrap(**{k: dev(v) for k, v in el.items()}),
+                                Arrays.wrap(**{k: dev(v) for k, v in prev.items()}))
+    torch.cuda.synchronize()
+    err = {k: relerr(host(getattr(out, k)), ref[k]) for k in ('px', 'py', 'dx_chaotic', 'dy_chaotic')}
+    print('  side', n, 'errors', {k: f'{v:.1e}' for k, v in err.items()})
+    assert max(err.values()) < 1e-12
+
+
 @pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
 def test_plasma_step_with_declustering_matches_oracle(precision):
     from lcodepy_amd.plasma3d.initialization import init_plasma
