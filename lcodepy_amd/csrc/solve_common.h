@@ -5,6 +5,8 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <type_traits>
+
 namespace lc3d {
 
 // Field order of the solve.
@@ -41,9 +43,23 @@ __device__ __forceinline__ double solver_factor(int f, int gr, int gc, int N, co
     return ok ? (1.0 / (sg.lam[gr] + sg.lam[gc] + cc)) / sg.d2 : 0.0;
 }
 
+// Calls g with the field f as a compile-time constant.
+template <typename G> __device__ __forceinline__ void with_field(int f, G g)
+{
+    switch (f) {
+    case F_EX: g(std::integral_constant<int, F_EX>{}); break;
+    case F_EY: g(std::integral_constant<int, F_EY>{}); break;
+    case F_BX: g(std::integral_constant<int, F_BX>{}); break;
+    case F_BY: g(std::integral_constant<int, F_BY>{}); break;
+    case F_EZ: g(std::integral_constant<int, F_EZ>{}); break;
+    case F_BZ: g(std::integral_constant<int, F_BZ>{}); break;
+    default: g(std::integral_constant<int, F_PHI>{}); break;
+    }
+}
+
 // Right-hand side of field f at (i, j) from the currents of layers k (P) and
 // k+1 (F), the beam densities and the predictor fields (fields.py:112-266).
-// Valid on in_rhs_domain(); the x/y stencils stay inside the grid there.
+// Valid on in_rhs_domain().
 template <typename TG, typename TPRED> struct RhsEval {
     SolveIn<TG, TPRED> in;
     int N;
@@ -63,36 +79,38 @@ template <typename TG, typename TPRED> struct RhsEval {
         return (jzF(o) + (TG)in.rbF[o] + jzP(o) + (TG)in.rbP[o]) * TG(0.5);
     }
 
-    __device__ TG operator()(int f, int i, int j) const {
+    // Loads are made for every (i, j) of the grid, at o itself where a stencil
+    // would leave it, so that none waits for a branch; the value outside
+    // in_rhs_domain() means nothing.
+    template <int F> __device__ __forceinline__ TG at(int i, int j) const {
         const int o = i * N + j;
         const bool inner = i > 0 && i < N - 1 && j > 0 && j < N - 1;
-        switch (f) {
-        case F_EX: {
-            const TG d = inner ? (ro_half(o + N) - ro_half(o - N)) * inv2h : TG(0);
+        const int dx = inner ? N : 0, dy = inner ? 1 : 0;
+        if constexpr (F == F_EX) {
+            const TG v = (ro_half(o + dx) - ro_half(o - dx)) * inv2h, d = inner ? v : TG(0);
             return -((d - (jxP(o) - jxF(o)) * invdxi) - c * (TG)in.ExP[o]);
-        }
-        case F_EY: {
-            const TG d = inner ? (ro_half(o + 1) - ro_half(o - 1)) * inv2h : TG(0);
+        } else if constexpr (F == F_EY) {
+            const TG v = (ro_half(o + dy) - ro_half(o - dy)) * inv2h, d = inner ? v : TG(0);
             return -((d - (jyP(o) - jyF(o)) * invdxi) - c * (TG)in.EyP[o]);
-        }
-        case F_BX: {
-            const TG d = inner ? (jz_half(o + 1) - jz_half(o - 1)) * inv2h : TG(0);
+        } else if constexpr (F == F_BX) {
+            const TG v = (jz_half(o + dy) - jz_half(o - dy)) * inv2h, d = inner ? v : TG(0);
             return (d - (jyP(o) - jyF(o)) * invdxi) + c * (TG)in.BxP[o];
-        }
-        case F_BY: {
-            const TG d = inner ? (jz_half(o + N) - jz_half(o - N)) * inv2h : TG(0);
+        } else if constexpr (F == F_BY) {
+            const TG v = (jz_half(o + dx) - jz_half(o - dx)) * inv2h, d = inner ? v : TG(0);
             return -((d - (jxP(o) - jxF(o)) * invdxi) - c * (TG)in.ByP[o]);
-        }
-        case F_EZ:
-            return -((jxF(o + N) - jxF(o - N)) + (jyF(o + 1) - jyF(o - 1))) * inv2h;
-        case F_BZ: {
-            const TG a = inner ? jxF(o + 1) - jxF(o - 1) : TG(0);
-            const TG b = inner ? jyF(o + N) - jyF(o - N) : TG(0);
-            return -(a - b) * inv2h;
-        }
-        default:   // F_PHI
+        } else if constexpr (F == F_EZ) {
+            return -((jxF(o + dx) - jxF(o - dx)) + (jyF(o + dy) - jyF(o - dy))) * inv2h;
+        } else if constexpr (F == F_BZ) {
+            const TG u = jxF(o + dy) - jxF(o - dy), v = jyF(o + dx) - jyF(o - dx);
+            return -((inner ? u : TG(0)) - (inner ? v : TG(0))) * inv2h;
+        } else {   // F_PHI
             return roF(o) - jzF(o);
         }
+    }
+    __device__ __forceinline__ TG operator()(int f, int i, int j) const {
+        TG r = TG(0);
+        with_field(f, [&](auto field) { r = at<decltype(field)::value>(i, j); });
+        return r;
     }
 };
 
