@@ -125,20 +125,52 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_cells(int ncell, int ntil
     __shared__ int sh[SCAN_THREADS / 64];
     int *__restrict__ count = bs.count;
     const int first = blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_PER;
-    int c[SCAN_PER];
+    // A thread's counts and starts are whole int4s, but at the end of the cells
+    // (word by word, each access of a wave touched 16 lines: N = 1025 19.7 -> 15.6
+    // us, 513 7.1 -> 5.4, 129 4.9 -> 3.2).  The rest at 1025 is the tiles' atomics;
+    // tiles of 4096 cells took 10 us there but 6.0 at 513 and 4.3 at 129.
+    const bool whole = first + SCAN_PER <= ncell;
+    int4 *__restrict__ count4 = reinterpret_cast<int4 *>(count + first);
+    int4 *__restrict__ lstart4 = reinterpret_cast<int4 *>(bs.lstart + first);
+    int c[SCAN_PER], start[SCAN_PER];
     int s = 0;
+    if (whole) {
 #pragma unroll
-    for (int i = 0; i < SCAN_PER; ++i) {
-        c[i] = first + i < ncell ? count[first + i] : 0;
-        s += c[i];
+        for (int i = 0; i < SCAN_PER / 4; ++i) {
+            const int4 v = count4[i];
+            c[4 * i] = v.x;
+            c[4 * i + 1] = v.y;
+            c[4 * i + 2] = v.z;
+            c[4 * i + 3] = v.w;
+            count4[i] = int4{0, 0, 0, 0};
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < SCAN_PER; ++i) {
+            c[i] = first + i < ncell ? count[first + i] : 0;
+            if (first + i < ncell) count[first + i] = 0;
+        }
     }
+#pragma unroll
+    for (int i = 0; i < SCAN_PER; ++i) s += c[i];
     int total;
     int run = block_exclusive_scan(s, sh, total);
 #pragma unroll
     for (int i = 0; i < SCAN_PER; ++i) {
-        if (first + i <= ncell) bs.lstart[first + i] = run;
-        if (first + i < ncell) count[first + i] = 0;
+        start[i] = run;
         run += c[i];
+    }
+    if (whole) {
+#pragma unroll
+        for (int i = 0; i < SCAN_PER / 4; ++i)
+            lstart4[i] = int4{start[4 * i], start[4 * i + 1], start[4 * i + 2], start[4 * i + 3]};
+    } else {
+#pragma unroll
+        for (int i = 0; i < SCAN_PER; ++i)
+            if (first + i <= ncell) bs.lstart[first + i] = start[i];
+    }
+#pragma unroll
+    for (int i = 0; i < SCAN_PER; ++i) {
         if (c[i] > SMALL_CELL) {
             // Two atomics, so that each is at one address and a wave's add as one.
             int slot;
