@@ -484,7 +484,7 @@ __global__ __launch_bounds__(RF_T) void k_rf_rows_fwd(RfftGeom g, RhsEval<TG, TP
             const int tr = dper.div(it), j = it - tr * per;
             const int ia = 2 * (p0 + tr), ib = min(ia + 1, N - 1);
             RF_CHECK(ia < N && j <= M);
-            const TG va = rhs.template at<F>(ia, j), vb = rhs.template at<F>(ib, j);
+            const TG va = rhs.template at<F, true>(ia, j), vb = rhs.template at<F, true>(ib, j);
             const TG a = in_rhs_domain(F, ia, j, N) ? va : TG(0);
             const TG b = ib > ia && in_rhs_domain(F, ib, j, N) ? vb : TG(0);
             C *t = lds + tr * RS;

@@ -79,37 +79,48 @@ template <typename TG, typename TPRED> struct RhsEval {
         return (jzF(o) + (TG)in.rbF[o] + jzP(o) + (TG)in.rbP[o]) * TG(0.5);
     }
 
-    // Loads are made for every (i, j) of the grid, at o itself where a stencil
-    // would leave it, so that none waits for a branch; the value outside
-    // in_rhs_domain() means nothing.
-    template <int F> __device__ __forceinline__ TG at(int i, int j) const {
+    // With ALL, loads are made for every (i, j) of the grid, at o itself where a
+    // stencil would leave it, so that none waits for a branch; the value outside
+    // in_rhs_domain() means nothing.  Without, under branches: the two may differ
+    // in the last bit (in what is fused into multiply-adds), and each kernel
+    // keeps to its form.
+    template <int F, bool ALL> __device__ __forceinline__ TG at(int i, int j) const {
         const int o = i * N + j;
         const bool inner = i > 0 && i < N - 1 && j > 0 && j < N - 1;
-        const int dx = inner ? N : 0, dy = inner ? 1 : 0;
+        const int dx = !ALL || inner ? N : 0, dy = !ALL || inner ? 1 : 0;
+        auto where_inner = [&](auto value) -> TG {
+            if constexpr (ALL) {
+                const TG v = value();
+                return inner ? v : TG(0);
+            } else {
+                return inner ? value() : TG(0);
+            }
+        };
         if constexpr (F == F_EX) {
-            const TG v = (ro_half(o + dx) - ro_half(o - dx)) * inv2h, d = inner ? v : TG(0);
+            const TG d = where_inner([&] { return (ro_half(o + dx) - ro_half(o - dx)) * inv2h; });
             return -((d - (jxP(o) - jxF(o)) * invdxi) - c * (TG)in.ExP[o]);
         } else if constexpr (F == F_EY) {
-            const TG v = (ro_half(o + dy) - ro_half(o - dy)) * inv2h, d = inner ? v : TG(0);
+            const TG d = where_inner([&] { return (ro_half(o + dy) - ro_half(o - dy)) * inv2h; });
             return -((d - (jyP(o) - jyF(o)) * invdxi) - c * (TG)in.EyP[o]);
         } else if constexpr (F == F_BX) {
-            const TG v = (jz_half(o + dy) - jz_half(o - dy)) * inv2h, d = inner ? v : TG(0);
+            const TG d = where_inner([&] { return (jz_half(o + dy) - jz_half(o - dy)) * inv2h; });
             return (d - (jyP(o) - jyF(o)) * invdxi) + c * (TG)in.BxP[o];
         } else if constexpr (F == F_BY) {
-            const TG v = (jz_half(o + dx) - jz_half(o - dx)) * inv2h, d = inner ? v : TG(0);
+            const TG d = where_inner([&] { return (jz_half(o + dx) - jz_half(o - dx)) * inv2h; });
             return -((d - (jxP(o) - jxF(o)) * invdxi) - c * (TG)in.ByP[o]);
         } else if constexpr (F == F_EZ) {
             return -((jxF(o + dx) - jxF(o - dx)) + (jyF(o + dy) - jyF(o - dy))) * inv2h;
         } else if constexpr (F == F_BZ) {
-            const TG u = jxF(o + dy) - jxF(o - dy), v = jyF(o + dx) - jyF(o - dx);
-            return -((inner ? u : TG(0)) - (inner ? v : TG(0))) * inv2h;
+            const TG a = where_inner([&] { return jxF(o + dy) - jxF(o - dy); });
+            const TG b = where_inner([&] { return jyF(o + dx) - jyF(o - dx); });
+            return -(a - b) * inv2h;
         } else {   // F_PHI
             return roF(o) - jzF(o);
         }
     }
     __device__ __forceinline__ TG operator()(int f, int i, int j) const {
         TG r = TG(0);
-        with_field(f, [&](auto field) { r = at<decltype(field)::value>(i, j); });
+        with_field(f, [&](auto field) { r = at<decltype(field)::value, false>(i, j); });
         return r;
     }
 };
