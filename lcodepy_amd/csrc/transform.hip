@@ -16,12 +16,12 @@
 //
 // Kernels, all on plain global buffers and static LDS:
 //   k_rhs       R of all seven fields (one thread per grid point, all fields);
-//   k_gemm_mfma C_f = A_f B_f for the seven fields of a launch (64 x 64
-//               tiles through LDS, 16x16x4 matrix-core products; the last
+//   k_gemm_mfma float32: C_f = A_f B_f for the seven fields of a launch (64 x
+//               64 tiles through LDS, 16x16x4 matrix-core products; the last
 //               row and column by the blocks of the last tile row and
 //               column), optionally scaled by M;
-//   k_gemm_split the same in float64 for the smaller N (16 x 16 or 32 x 32
-//               tiles, k split over the waves);
+//   k_gemm_split the same in float64 (16 x 16 or 32 x 32 tiles, k split over
+//               the waves);
 //   k_assemble  outputs (full / half fields) and the Bz row sums;
 //   k_bz_finalize  mean of Bz removed, half-step Bz.
 #include "mfma.h"
@@ -53,14 +53,13 @@ __global__ __launch_bounds__(256) void k_rhs(RhsEval<TG, TPRED> rhs, TG *__restr
 }
 
 constexpr int GBM = 64, GBN = 64;   // output tile
-// The float64 product: 16 x 16 split tiles below GEMM_SMALL, 32 x 32 split
-// tiles below GEMM_SPLIT, k_gemm_mfma from there on (k_gemm_split).
-constexpr int GEMM_SMALL = 200, GEMM_SPLIT = 336;
+// The float64 product: 16 x 16 tiles below GEMM_SMALL, 32 x 32 from there on
+// (k_gemm_split).
+constexpr int GEMM_SMALL = 200;
 constexpr int GTJ = GBN / 32;       // 16-column products per wave (waves 2 x 2)
-// Depth of a k tile: 64 in float32, 32 in float64 (two blocks per CU fit
-// the double-buffered LDS tiles either way).
+// k tiles are 64 deep (two blocks per CU fit the double-buffered LDS tiles).
 template <typename T> struct GemmTile {
-    static constexpr int BK = sizeof(T) == 4 ? 64 : 32;
+    static constexpr int BK = 64;
     static constexpr int RS = BK + 4;            // LDS row stride of the A and B^T tiles
     static constexpr int NA = GBM * BK / 256;    // A elements per thread per tile
     static constexpr int NB = BK * GBN / 256;    // B elements per thread per tile
@@ -255,18 +254,19 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mfma(GemmBatch<T> bt, int N, Sc
 // tile is (16 R) x (16 R) output elements, and wave w sums k in its quarter of
 // [0, N) for the whole tile, its operands straight from memory into the
 // matrix cores' registers (the next 16 k in flight), so that nothing waits at
-// a barrier before the four partial tiles meet in LDS.  The 64 x 64 tiles of
-// k_gemm_mfma give N = 129 28 blocks and N = 321 175, each a serial chain of k
-// tiles; float32 keeps them, where the order of the k sum decides the result
-// at its precision.  Measured per solve (four products and the passes around
-// them; 16 x 16 split, 32 x 32 split, k_gemm_mfma; us): N = 65 26, 30, 53; 129
-// 36, 39, 73; 193 57, 62, 98; 225 77, 68, 97; 257 92, 91, 115; 321 161, 134, 140;
-// 385 247, 189, 169; 513 482, 333, 293: the split tiles read (N / 16 R)^2 N of
-// both operands past the L2 at about 6.8 TB/s, which bounds them from N of
-// about 300.
-// Lane l of a wave takes k = kk + 4 (l / 16) + s in step s of a group of 16, the
-// same for A and B, so that it reads four neighbouring elements of A's row.
-// Rows, columns and k beyond the matrix read its last ones and count zero.
+// a barrier before the four partial tiles meet in LDS.  Lane l of a wave takes
+// k = kk + 4 (l / 16) + s in step s of a group of 16, the same for A and B, so
+// that it reads four neighbouring elements of A's row, two at a time: one by
+// one, four accesses went to every line (N = 129 36 us a solve, 321 134, 385 189,
+// 513 333), the rest of which the L1 no longer held.
+// Measured per solve (four products and the passes around them; 16 x 16, 32 x
+// 32, and the 64 x 64 tiles of k_gemm_mfma in float64; us): N = 65 24, 31, 53;
+// 129 32, 35, 73; 161 37, 37, 77; 193 48, 53, 97; 225 61, 58, 97; 257 72, 76, 114;
+// 321 122, 105, 141; 385 177, 143, 166; 513 336, 240, 279; 769 1179, 699, 771; 1025
+// 2695, 1476, 1675 (48 x 48: 118 at 321, 271 at 513, 690 and 1377 at the last two).
+// Float32 keeps the 64 x 64 tiles, where the order of the k sum decides the
+// result at its precision.
+// Rows and columns beyond the matrix read its last ones; k beyond it counts zero.
 template <typename T, int R, bool SCALE>
 __global__ __launch_bounds__(256) void k_gemm_split(GemmBatch<T> bt, int N, ScaleGeom sg)
 {
@@ -300,20 +300,37 @@ __global__ __launch_bounds__(256) void k_gemm_split(GemmBatch<T> bt, int N, Scal
         for (int j = 0; j < R; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[i][j][r] = T(0);
+    // 16 values of k at a time, four consecutive ones a lane; the last of the
+    // range may be part of them.
     T a[2][R][4], b[2][R][4];
+    struct Two {
+        T x, y;   // aligned as one value
+    };
     auto load = [&](auto set, int kk) {
         constexpr int S = decltype(set)::value;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const Two *p = reinterpret_cast<const Two *>(pa[r] + kk + 4 * lk);
+            const Two u = p[0], v = p[1];
+            a[S][r][0] = u.x;
+            a[S][r][1] = u.y;
+            a[S][r][2] = v.x;
+            a[S][r][3] = v.y;
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int r = 0; r < R; ++r) b[S][r][s] = pb[r][(size_t)(kk + 4 * lk + s) * N];
+    };
+    auto load_part = [&](int kk) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int k = kk + 4 * lk + s, kc = min(k, N - 1);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                a[S][r][s] = pa[r][kc];
-                b[S][r][s] = pb[r][(size_t)kc * N];
-            }
-            if (k >= k1) {
-#pragma unroll
-                for (int r = 0; r < R; ++r) a[S][r][s] = b[S][r][s] = T(0);
+                const T u = pa[r][kc], v = pb[r][(size_t)kc * N];
+                a[0][r][s] = k < k1 ? u : T(0);
+                b[0][r][s] = k < k1 ? v : T(0);
             }
         }
     };
@@ -328,14 +345,17 @@ __global__ __launch_bounds__(256) void k_gemm_split(GemmBatch<T> bt, int N, Scal
     };
     using Zero = std::integral_constant<int, 0>;
     using One = std::integral_constant<int, 1>;
-    if (k0 < k1) {   // whole waves
-        load(Zero{}, k0);
-        for (int kk = k0; kk < k1; kk += 32) {
-            if (kk + 16 < k1) load(One{}, kk + 16);
-            multiply(Zero{});
-            if (kk + 32 < k1) load(Zero{}, kk + 32);
-            if (kk + 16 < k1) multiply(One{});
-        }
+    const int kf = k0 + (k1 - k0) / 16 * 16;   // k0 .. kf in whole sixteens
+    if (k0 < kf) load(Zero{}, k0);
+    for (int kk = k0; kk < kf; kk += 32) {
+        if (kk + 16 < kf) load(One{}, kk + 16);
+        multiply(Zero{});
+        if (kk + 32 < kf) load(Zero{}, kk + 32);
+        if (kk + 16 < kf) multiply(One{});
+    }
+    if (kf < k1) {
+        load_part(kf);
+        multiply(Zero{});
     }
 #pragma unroll
     for (int i = 0; i < R; ++i)
@@ -369,11 +389,12 @@ void gemm_launch(const GemmBatch<T> &bt, int N, const ScaleGeom &sg, hipStream_t
     static_assert(GemmTile<T>::BK <= 64, "the edge loaders use threads 0..127");
     static_assert(GBN % 32 == 0 && GBN <= 64 && GBM == 64, "wave layout 2 x 2");
     if constexpr (std::is_same<T, double>::value) {
-        if (N < GEMM_SMALL) return gemm_split_launch<T, 1, SCALE>(bt, N, sg, s);
-        if (N < GEMM_SPLIT) return gemm_split_launch<T, 2, SCALE>(bt, N, sg, s);
+        if (N < GEMM_SMALL) gemm_split_launch<T, 1, SCALE>(bt, N, sg, s);
+        else gemm_split_launch<T, 2, SCALE>(bt, N, sg, s);
+    } else {
+        const dim3 grid((N - 1 + GBN - 1) / GBN, (N - 1 + GBM - 1) / GBM, 7);
+        k_gemm_mfma<T, SCALE><<<grid, 256, 0, s>>>(bt, N, sg);
     }
-    const dim3 grid((N - 1 + GBN - 1) / GBN, (N - 1 + GBM - 1) / GBM, 7);
-    k_gemm_mfma<T, SCALE><<<grid, 256, 0, s>>>(bt, N, sg);
 }
 
 // One wave per (row, field): outputs of the row and, for Bz, its row sum.
