@@ -143,15 +143,17 @@ uint64_t rfft_default_plan(int L)
 // for more waves a SIMD and spill.  Measured (default plan, us per solve,
 // this shape against filling the largest LDS size): float32 N = 129 29 (68),
 // 257 39 (76), 417 72 (97), 513 78 (101), 1025 278 (388); float64 129 32 (50),
-// 257 48 (59), 385 94 (101), 513 133, 1025 496.
+// 257 48 (59), 385 94 (101), 513 133, 1025 496.  Float64 transforms of 513 to 682
+// points fill the largest LDS size with three (N = 337 74 us; one a block 82).
 void rfft_default_shape(int L, bool f32, int &cap, int &tpb)
 {
     if (f32) {
         cap = L > 512 && L < 1024 ? 2048 : 4096;
         tpb = L == 1024 ? 2 : 1;
     } else {
-        cap = (L > 256 && L < 512) || (L > 640 && L < 1024) ? 2048 : 4096;
-        tpb = L == 512 || L == 1024 ? 2 : L > 512 && L <= 640 ? 4096 / (2 * L) : 1;
+        constexpr int three = 4096 / 6;   // the longest of which three fit a block
+        cap = (L > 256 && L < 512) || (L > three && L < 1024) ? 2048 : 4096;
+        tpb = L == 512 || L == 1024 ? 2 : L > 512 && L <= three ? 4096 / (2 * L) : 1;
     }
 }
 
