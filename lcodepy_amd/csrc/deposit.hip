@@ -17,8 +17,9 @@
 //               their ranks; the ids are the cell order the next push visits
 //               (so binning positions follow the cell order, and a cell's
 //               records lie close together);
-//   4. dense    per dense cell its list sorted by particle id and its 5 x 5 x 4
-//               taps, by one workgroup with a fixed-order reduction;
+//   4. dense    per dense cell its list in particle-id order and its 5 x 5 x 4
+//               taps, by a wave, four waves or a workgroup with a fixed-order
+//               reduction;
 //   5. gather   one workgroup per tile of output cells sorts the lists of the
 //               source cells around it by particle id, stages their records
 //               in LDS and sums them, every output cell in a fixed order.

@@ -285,6 +285,52 @@ def test_deposit_of_cells_at_the_edges_of_the_lists(N, precision):
         assert relerr(host(u[0]), w) < (3e-5 if f32 else 1e-12)
 
 
+@pytest.mark.parametrize('N', [641, 653])
+def test_float32_deposit_on_both_sides_of_the_larger_tiles(N):
+    """The same lists in float32 at the grids between which it takes tiles of
+    eight rows (float64 does between 433 and 449)."""
+    test_deposit_of_cells_at_the_edges_of_the_lists(N, 'fp32-bulk')
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
+@pytest.mark.parametrize('lengths', [(17, 63, 64, 65), (128, 255, 256, 257), (64, 65, 512, 513, 1025)])
+def test_deposit_of_dense_cells_at_the_edges_of_their_lists(lengths, precision):
+    """Dense cells on both sides of each list length that one wave, four waves
+    or a workgroup sorts and sums, an odd number of the longer ones (two are a
+    workgroup's at a time), visited in random order.  A density sums up to 25
+    cells of the longest list, in trees of about 40 roundings, of which a tenth
+    may be left by cancellation: 1e-12 of the maximum in float64, 3e-5 in
+    float32."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.weights import get_deposit_plasma
+    print(f'dense lists {lengths} {precision}', flush=True)
+    f32 = precision == 'fp32-bulk'
+    N, fineness = 65, 5
+    rng = np.random.default_rng(lengths[0] + lengths[-1])
+    p = _params(N, fineness=fineness)
+    count = np.zeros(N * N, dtype=int)
+    inner = np.arange(N * N).reshape(N, N)[8:N - 8, 8:N - 8].ravel()
+    some = rng.choice(inner, 41, replace=False)
+    count[some] = np.resize(lengths, some.size)
+    cell = rng.permutation(np.repeat(np.arange(N * N), count))
+    n = cell.size
+    at = lambda k: (k - N // 2 + 0.98 * rng.uniform(-0.5, 0.5, n)) * p.h
+    m = np.full(n, 0.01)
+    a = dict(x_init=at(cell // N), y_init=at(cell % N), x_offt=np.zeros(n), y_offt=np.zeros(n),
+             q=-m, m=m, **{k: m * rng.normal(0, 0.1, n) for k in ('px', 'py', 'pz')})
+    if f32:
+        a = _round_bulk(a)
+    g = [np.zeros((N, N)) for _ in range(4)]
+    O.deposit_sort(p, a, *g)
+    deposit = get_deposit_plasma(_cfg(N, precision=precision, fineness=fineness))
+    const = Arrays.wrap()
+    const.sorts = {'electrons': 0}
+    out = deposit({'electrons': _sort_arrays(a, torch.float32 if f32 else torch.float64)}, const)
+    torch.cuda.synchronize()
+    for u, w in zip(out, g):
+        assert relerr(host(u[0]), w) < (3e-5 if f32 else 1e-12)
+
+
 @pytest.mark.parametrize('N,frac', [(65, 0.005), (65, 0.05), (65, 0.3), (129, 0.45)])
 def test_deposit_of_collapsed_plasma(N, frac):
     """A fraction of the particles collapsed into the cell on the axis
