@@ -292,7 +292,7 @@ __device__ __forceinline__ int wave_value(int lane)
 template <typename T>
 __global__ __launch_bounds__(DENSE_BLOCK) void k_dense_cells(double h, BinState bs)
 {
-    __shared__ unsigned long long s[MAX_SORTED_CELL];   // particle id << 32 | position
+    __shared__ __align__(16) unsigned long long s[MAX_SORTED_CELL];   // particle id << 32 | position
     __shared__ T red[DENSE_WAVES][PAIR_VALUES];
     const int few = min(bs.nbig[0], bs.bigcap), many = min(bs.nbig[1], bs.bigcap - few);
     const DepRec<T> *__restrict__ rec = static_cast<const DepRec<T> *>(bs.rec);
