@@ -1,13 +1,11 @@
 """Beam layer calculators (beam3d/beam_calculator.py:60-181)."""
 from __future__ import annotations
 
-import ctypes
-
 from .. import runtime
 from .._native import BeamRows, ptr, stream_ptr
 from ..config import Config
 from ..plasma3d import _bind
-from .data import BeamParticles, empty_rounded
+from .data import FLOAT_KEYS, INT_KEYS, BeamParticles, empty_rounded
 from .move import get_move_beam_particles
 from .weights import get_deposit_beam
 
@@ -81,6 +79,7 @@ class BeamCalculator:
         n, dev = beam_layer.size, runtime.device()
         if n == 0:
             return PendingMove(None, None, None, None)
+        _check_columns(beam_layer)
         beam_layer.contiguous()
         # lost, moved, fell: every entry is written by the move
         flags = empty_rounded((3, n), torch.uint8, dev)
@@ -104,11 +103,19 @@ class BeamCalculator:
                             fields_after_layer, fields_before_layer) -> 'PendingMove':
         """:meth:`move_beam_layer_async` of ``layer`` followed by the particles
         ``fell`` into it, in one library call that reads both where they are
-        (column slices of packed rows included) and changes neither."""
+        (column slices of packed rows included) and changes neither.  Layers
+        that are not packed rows are joined and go through that method."""
         import torch
         n, dev = layer.size + fell.size, runtime.device()
         if n == 0:
             return PendingMove(None, None, None, None)
+        rows = [_beam_rows(b) for b in (layer, fell)]
+        if None in rows:
+            joined = BeamParticles().append(layer).append(fell)
+            if joined.f is layer.f or joined.f is fell.f:
+                joined = BeamParticles(f=joined.f.clone(), i=joined.i.clone())
+            return self.move_beam_layer_async(joined, fell.size, pl_layer_idx,
+                                              fields_after_layer, fields_before_layer)
         for f in (fields_after_layer, fields_before_layer):
             if f.Ex.dtype.itemsize != 8:
                 raise TypeError('the beam moves in the float64 fields of layers k and k+1')
@@ -117,7 +124,6 @@ class BeamCalculator:
         out_f = empty_rounded((3, 9, n), torch.float64, dev)
         out_i = empty_rounded((3, 2, n), torch.int64, dev)
         counts_dev = torch.empty(3, dtype=torch.int64, device=dev)
-        rows = [_beam_rows(b) for b in (layer, fell)]
         self.ctx.check(self.ctx.lib.lc3d_beam_advance(
             self.ctx.handle, rows[0], rows[1], int(pl_layer_idx) - 1, self.substep_energy,
             self.time_step, _bind.fields6(fields_after_layer), _bind.fields6(fields_before_layer),
@@ -134,18 +140,27 @@ class BeamCalculator:
         return beam_layer_to_move, fell_to_next_layer.size, ro_beam_full.clone()
 
 
-def _beam_rows(b: BeamParticles) -> BeamRows:
-    """The packed rows of a layer as they are; rows whose columns are not
-    neighbours are copied first."""
-    if b.size == 0:
+def _check_columns(b: BeamParticles) -> None:
+    """The kernels take as many 8-byte columns of ``i`` as of ``f``."""
+    if b.f.dtype.itemsize != 8 or b.i.dtype.itemsize != 8:
+        raise TypeError(f'a beam layer is float64 and int64 rows, got {b.f.dtype} and {b.i.dtype}')
+    if b.i.shape[1] != b.f.shape[1]:
+        raise ValueError(f'a beam layer of {b.f.shape[1]} particles with {b.i.shape[1]} ids')
+
+
+def _beam_rows(b: BeamParticles) -> BeamRows | None:
+    """The packed rows of a layer as they are, or None if they are not what
+    lc3d_beam_advance reads: nine float64 and two int64 rows on the device,
+    the columns of each next to each other and no row over another."""
+    n = b.size
+    if n == 0:
         return BeamRows(0, None, 0, None, 0)
-    f, i = b.f, b.i
-    if f.stride(1) != 1 or i.stride(1) != 1:
-        b.contiguous()
-        f, i = b.f, b.i
-    if not (f.is_cuda and i.is_cuda) or f.dtype.itemsize != 8 or i.dtype.itemsize != 8:
-        raise TypeError('a beam layer is float64 and int64 rows on the device')
-    return BeamRows(f.shape[1], f.data_ptr(), f.stride(0), i.data_ptr(), i.stride(0))
+    _check_columns(b)
+    for t, count in ((b.f, len(FLOAT_KEYS)), (b.i, len(INT_KEYS))):
+        if (t.shape[0] != count or not t.is_cuda or (n > 1 and t.stride(1) != 1)
+                or t.stride(0) < n):
+            return None
+    return BeamRows(n, b.f.data_ptr(), b.f.stride(0), b.i.data_ptr(), b.i.stride(0))
 
 
 class PendingMove:

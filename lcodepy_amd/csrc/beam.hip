@@ -369,11 +369,15 @@ __global__ __launch_bounds__(BEAM_THREADS) void k_beam_advance(BeamGeom g, BeamR
         const int64_t fs = from.f_stride;
         const int64_t *iv = from.i + c;
         const double qm = f[BF_QM * fs];
-        double dt = f[BF_DT * fs];
+        double dt;
         BeamState b{f[BF_X * fs],  f[BF_Y * fs],  f[BF_XI * fs],
-                    f[BF_PX * fs], f[BF_PY * fs], f[BF_PZ * fs],
-                    iv[BI_STEPS * from.i_stride], false, false, false};
-        if (laid) substeps_of(qm, b.pz, e_sub, time_step, dt, b.steps);
+                    f[BF_PX * fs], f[BF_PY * fs], f[BF_PZ * fs], 0, false, false, false};
+        if (laid) {
+            substeps_of(qm, b.pz, e_sub, time_step, dt, b.steps);
+        } else {   // its substeps go on
+            dt = f[BF_DT * fs];
+            b.steps = iv[BI_STEPS * from.i_stride];
+        }
         move_particle<TF>(g, xi_k, xi_k1, qm, dt, fk, fk1, lane, b);
         if (b.off) atomicOr(err, ERR_BEAM_OFF_GRID);
         if (lane == 0) {

@@ -1,4 +1,5 @@
-"""Host-side beam bookkeeping on CPU tensors: the drain's periodic joining
+"""Host-side beam bookkeeping on CPU tensors: a layer whose rows are not what
+the move reads never reaches the library; the drain's periodic joining
 keeps the order of the layers pushed (beam3d/beam_io.py:50-73, whose drain
 appends every layer to its buffer as it arrives), and buffers rounded to a power of
 two are ordinary contiguous tensors of the asked shape."""
@@ -51,3 +52,45 @@ def test_append_into_rounded_buffer_keeps_values():
     assert a.size == 5
     assert torch.equal(a.id, torch.tensor([1, 2, 3, 10, 11]))
     assert a.f.is_contiguous()
+
+
+class _Refuses:
+    """A library whose entry points must not be called."""
+
+    def __getattr__(self, name):
+        def call(*args):
+            raise AssertionError(f'{name} was called')
+        return call
+
+
+@pytest.mark.parametrize('float_rows,int_rows,ids,dtype,error', [
+    (8, 2, 5, torch.float64, IndexError), (6, 2, 5, torch.float64, IndexError),
+    (9, 1, 5, torch.float64, IndexError), (9, 2, 4, torch.float64, ValueError),
+    (9, 2, 6, torch.float64, ValueError), (9, 2, 5, torch.float32, TypeError)])
+@pytest.mark.parametrize('part', ['layer', 'fell'])
+def test_advance_refuses_rows_it_would_read_past(monkeypatch, part, float_rows, int_rows, ids,
+                                                 dtype, error):
+    """A layer without all its rows (or with fewer or more ids than columns)
+    raises what indexing the missing row raises, before any kernel gets its
+    address (beam_calculator.py:97-143)."""
+    from types import SimpleNamespace
+
+    from lcodepy_amd import runtime
+    from lcodepy_amd.beam3d import beam_calculator, move
+    monkeypatch.setattr(torch.Tensor, 'is_cuda', property(lambda t: True))
+    monkeypatch.setattr(runtime, 'device', lambda: torch.device('cpu'))
+    monkeypatch.setattr(beam_calculator, 'stream_ptr', lambda: 0)
+    ctx = SimpleNamespace(lib=_Refuses(), handle=None, check=None)
+    monkeypatch.setattr(runtime, 'context', lambda config: ctx)
+    calc = beam_calculator.BeamCalculator.__new__(beam_calculator.BeamCalculator)
+    calc.ctx, calc.substep_energy, calc.time_step = ctx, 2.0, 1.0
+    calc.move_particles = move.get_move_beam_particles(None)
+    fields = SimpleNamespace(**{k: torch.zeros(3, 3, dtype=torch.float64)
+                                for k in ('Ex', 'Ey', 'Ez', 'Bx', 'By', 'Bz')})
+    wrong = BeamParticles(f=torch.zeros(float_rows, 5, dtype=dtype),
+                          i=torch.zeros(int_rows, ids, dtype=torch.int64))
+    none = BeamParticles(f=torch.zeros(9, 0, dtype=torch.float64),
+                         i=torch.zeros(2, 0, dtype=torch.int64))
+    layer, fell = (wrong, none) if part == 'layer' else (none, wrong)
+    with pytest.raises(error):
+        calc.advance_layer_async(layer, fell, 4, fields, fields)

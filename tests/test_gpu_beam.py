@@ -165,6 +165,46 @@ def test_beam_advance_equals_the_separate_calls(n_layer, n_fell):
         assert torch.equal(g.f, w.f) and torch.equal(g.i, w.i)
 
 
+@pytest.mark.parametrize('layout', ['ten rows', 'every other column', 'one row for all', 'one'])
+def test_beam_advance_of_rows_laid_out_otherwise(layout):
+    """A layer of ten float rows (the tenth goes with its particles), of
+    columns that are not neighbours, with one row shared by all (an expanded
+    tensor), and of one particle with strides of its own gives what the
+    separate calls give for contiguous rows, bit for bit (the same kernels),
+    and is left as it is."""
+    from lcodepy_amd.beam3d.beam_calculator import BeamCalculator
+    from lcodepy_amd.beam3d.data import FLOAT_KEYS, INT_KEYS, BeamParticles
+    from lcodepy_amd.plasma3d.data import Arrays
+    print(f'beam advance: {layout}', flush=True)
+    rng = np.random.default_rng(5)
+    b = _layer(rng)
+    f = torch.tensor(np.stack([b[k] for k in FLOAT_KEYS]), device='cuda')
+    i = torch.tensor(np.stack([b[k] for k in INT_KEYS]), device='cuda')
+    i[0] = torch.arange(1, i.shape[1] + 1, device='cuda')
+    if layout == 'ten rows':
+        f = torch.cat((f, f[:1] * 3))
+    elif layout == 'every other column':
+        f, i = f[:, ::2], i[:, ::2]
+    elif layout == 'one row for all':
+        f = f[7].expand(9, -1)
+    else:
+        f, i = f[:, 3:4].t().contiguous().t(), i[:, 3:4]
+    layer, fell = BeamParticles(f=f, i=i), BeamParticles()
+    before = f.clone(), i.clone()
+    fields = [Arrays.wrap(**{k: torch.tensor(_smooth(rng, 0.05), device='cuda')
+                             for k in ('Ex', 'Ey', 'Ez', 'Bx', 'By', 'Bz')}) for _ in range(2)]
+    calc = BeamCalculator(_config())
+    got = calc.advance_layer_async(layer, fell, LAYER, *fields).result()
+    assert torch.equal(layer.f, before[0]) and torch.equal(layer.i, before[1])
+    joined = BeamParticles(f=before[0].contiguous(), i=before[1].contiguous())
+    want = calc.move_beam_layer(joined, 0, LAYER, *fields)
+    calc.ctx.raise_on_errors()
+    assert sum(g.size for g in got) >= layer.size
+    for g, w in zip(got, want):
+        assert g.f.shape[0] == f.shape[0]
+        assert torch.equal(g.f, w.f) and torch.equal(g.i, w.i)
+
+
 @pytest.mark.parametrize('n', [1, 700, 1024, 5000, 32 * 1024, 40000])
 def test_beam_split_keeps_layer_order(n):
     """lc3d_beam_split (beam_calculator.py:124-139) against numpy's boolean
