@@ -116,6 +116,29 @@ template <typename TP, typename TG, typename TH> void run_all(int N, int prec, i
     CHECK(lc3d_beam_substep(r.ctx, nb, bqm, bpz, 2.0, 1.0, bdt, bst, nullptr));
     lc3d_fields6 fk{full.Ex, full.Ey, full.Ez, full.Bx, full.By, full.Bz};
     CHECK(lc3d_move_beam(r.ctx, nb, 3, bqm, bdt, &fk, &fk, bst, bid, bx, by, bxi, bpx, bpy, bpz, l, mv, fl, nullptr));
+    // one layer's advance: the layer's columns start at 3 of wider rows and are
+    // its rows' last, the fallen particles' at 0; outputs and scratch exactly sized
+    {
+        const int64_t nl = 75, nf = 22, na = nl + nf, fs = nl + 3;
+        double *lf = arr<double>(9 * fs), *ff = arr<double>(9 * nf), *of = arr<double>(27 * na);
+        int64_t *li = arr<int64_t>(2 * fs), *fi = arr<int64_t>(2 * nf), *oi = arr<int64_t>(6 * na), *cnt = arr<int64_t>(3);
+        auto fill = [&](double *f, int64_t *i, int64_t w, int64_t from, int64_t n) {
+            for (int64_t k = from; k < from + n; ++k) {
+                f[k] = -0.2 + uni(-0.05, 0); f[w + k] = 0.5 * nrm(); f[2 * w + k] = 0.5 * nrm();
+                f[5 * w + k] = k % 7 == 0 ? 1.0 : 1000.0; f[6 * w + k] = -1; f[7 * w + k] = 0.01;
+                f[8 * w + k] = 0.5; i[k] = k + 1; i[w + k] = 2;
+            }
+        };
+        fill(lf, li, fs, 3, nl); fill(ff, fi, nf, 0, nf);
+        const int64_t bytes = LC3D_BEAM_ADVANCE_SCRATCH(na);
+        double *sc = (double *)arr<uint8_t>(bytes);
+        lc3d_beam_rows layer{nl, lf + 3, fs, li + 3, fs}, fell{nf, ff, nf, fi, nf}, none{0, nullptr, 0, nullptr, 0};
+        CHECK(lc3d_beam_advance(r.ctx, &layer, &fell, 3, 2.0, 1.0, &fk, &fk, sc, bytes, of, oi, cnt, nullptr));
+        if (cnt[0] + cnt[1] + cnt[2] < na) { printf("FAIL beam advance lost particles\n"); exit(1); }
+        CHECK(lc3d_beam_advance(r.ctx, &none, &fell, 3, 2.0, 1.0, &fk, &fk, sc, bytes, of, oi, cnt, nullptr));
+        CHECK(lc3d_beam_advance(r.ctx, &none, &none, 3, 2.0, 1.0, &fk, &fk, nullptr, 0, nullptr, nullptr, nullptr, nullptr));
+        if (lc3d_beam_advance(r.ctx, &layer, &fell, 3, 2.0, 1.0, &fk, &fk, sc, bytes - 1, of, oi, cnt, nullptr) != LC3D_EINVAL) { printf("FAIL beam advance scratch check\n"); exit(1); }
+    }
     uint32_t flags = 0; CHECK(lc3d_error_flags(r.ctx, &flags, nullptr));
     printf("beam ok, error flags %u\n", flags); fflush(stdout);
     // energy flux: the context entry and the allocation-free one (static scratch)

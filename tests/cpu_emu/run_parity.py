@@ -72,6 +72,9 @@ class _DoneEvent:
     def synchronize(self):
         pass
 
+    def query(self):
+        return True
+
 
 torch.cuda.Event = _DoneEvent
 

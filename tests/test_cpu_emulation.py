@@ -86,3 +86,30 @@ def test_gpu_parity_suite_on_cpu_build(emu_build):
                        capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
     assert 'ERROR: AddressSanitizer' not in r.stderr
+
+
+@pytest.mark.parametrize('ids', [
+    # the particle-beam loop and the kernels of one layer's advance
+    ['tests/test_gpu_simulation.py::test_short_beam_evolution_matches_oracle',
+     'tests/test_gpu_beam.py::test_beam_advance_equals_the_separate_calls',
+     'tests/test_gpu_beam.py::test_beam_advance_of_rows_laid_out_otherwise'],
+    # dense cells by a wave, four waves and a workgroup; the gather's list lengths
+    ['tests/test_gpu_kernels.py::test_deposit_of_dense_cells_at_the_edges_of_their_lists[lengths0-fp64]',
+     'tests/test_gpu_kernels.py::test_deposit_of_dense_cells_at_the_edges_of_their_lists[lengths1-fp32-bulk]',
+     'tests/test_gpu_kernels.py::test_deposit_of_dense_cells_at_the_edges_of_their_lists[lengths2-fp64]',
+     'tests/test_gpu_kernels.py::test_deposit_of_cells_at_the_edges_of_the_lists[65-fp64]'],
+    # the staged push, both tiles of the float64 products, the smoothing's ends
+    ['tests/test_gpu_kernels.py::test_push_does_not_depend_on_how_particles_are_visited[65537-fp64]',
+     'tests/test_gpu_kernels.py::test_float64_matrix_solve_at_the_edges_of_its_tiles[199]',
+     'tests/test_gpu_kernels.py::test_float64_matrix_solve_at_the_edges_of_its_tiles[201]',
+     'tests/test_gpu_declustering.py::test_noise_filter_of_few_and_of_all_taps'],
+], ids=['beam', 'dense', 'staged'])
+def test_more_gpu_parity_tests_on_cpu_build(emu_build, ids):
+    """The paths that only larger inputs or a moving beam reach, a process of
+    their own per group."""
+    env = _env()
+    env['LD_PRELOAD'] = _libasan()
+    r = subprocess.run(['python3', os.path.join(EMU, 'run_parity.py')] + ids,
+                       capture_output=True, text=True, env=env, timeout=600)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+    assert 'ERROR: AddressSanitizer' not in r.stderr

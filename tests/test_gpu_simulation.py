@@ -188,3 +188,31 @@ def test_evolving_beam_runs_are_bitwise_equal():
     assert runs[0]['beam_id'].numel() > 0
     for k in runs[0]:
         assert torch.equal(runs[0][k], runs[1][k]), k
+
+
+def test_short_beam_evolution_matches_oracle():
+    """Two time steps of eight layers of a small window: the same loop at a
+    size that the host build runs too (every layer's deposit, advance and
+    drain).  Bounds as of the longer run above."""
+    from lcodepy_amd.beam_generator import generate_beam
+    from lcodepy_amd.simulation import Simulation
+    cfg = fixture_config('beam_evol')
+    cfg.update({'window-width': 2.4, 'transverse-step': 0.1, 'window-length': 0.4,
+                'time-limit': 2, 'time-step': 1})
+    beam_params = {'current': 0.5, 'particles_in_layer': 1000}
+    c = adjusted(cfg)
+    p = O.Params.from_config(c)
+    _, _, _, beam_o, ez_o = O.simulate(p, generate_beam(c, beam_params), 2)
+    sim = Simulation(config=cfg, beam_parameters=beam_params, runas_filename='')
+    sim.push_solver.verbose = False
+    sim.step()
+    drained = sim.beam_drain.beam_slice()
+    ids = drained.id.cpu().numpy()
+    order_g, order_o = np.argsort(ids), np.argsort(beam_o['id'])
+    print(f'N={p.N}: {len(ids)} drained particles (oracle {len(beam_o["id"])})', flush=True)
+    assert len(ids) > 0
+    assert np.array_equal(ids[order_g], beam_o['id'][order_o])
+    for k in ('x', 'y', 'xi', 'px', 'py', 'pz'):
+        assert relerr(getattr(drained, k).cpu().numpy()[order_g], beam_o[k][order_o]) < 1e-9, k
+    ez_g = np.array([float(v) for v in sim.push_solver.ez_axis])
+    assert relerr(ez_g, ez_o) < 1e-9
