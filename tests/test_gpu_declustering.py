@@ -129,3 +129,33 @@ def test_plasma_step_with_declustering_matches_oracle(precision):
     bound = 1e-4 if precision == 'fp32-bulk' else 1e-11
     for k, v in err.items():
         assert v < bound, (k, v)
+
+
+def test_noise_filter_of_a_lattice_whose_rows_take_most_lds():
+    """Smoothing by taps over the whole period of a lattice side at which a row
+    unrolled to what the outputs read takes more than 64 KB of LDS.  Some
+    thousand products a direction, in a running sum: 1e-12 of the maximum."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.noise_filter import get_noise_filter
+    N, fineness = 961, 4
+    cfg = _cfg(N, fineness=fineness)
+    for k, v in (('enabled', True), ('averaging', 2), ('force', 0.3), ('limit', 1e-3)):
+        cfg.set('declustering-' + k, v)
+    p = _params(N, fineness=fineness)
+    p.declustering = O.Declustering(averaging=2, force=0.3, damping=0.0, limit=1e-3)
+    el = O.uniform_plasma(p)
+    n = el['x_offt'].shape[0]
+    print(f'noise filter N={N} side {n}', flush=True)
+    rng = np.random.default_rng(N)
+    for k in ('x_offt', 'y_offt'):
+        el[k] = 3e-4 * rng.standard_normal((n, n))
+    for k in ('px', 'py', 'pz'):
+        el[k] = 1e-3 * rng.standard_normal((n, n))
+    prev = {k: 1e-4 * rng.standard_normal((n, n)) for k in ('dx_chaotic', 'dy_chaotic')}
+    ref = O.noise_filter(p, {k: v.copy() for k, v in el.items()}, prev)
+    out = get_noise_filter(cfg)(Arrays.wrap(**{k: dev(v) for k, v in el.items()}),
+                                Arrays.wrap(**{k: dev(v) for k, v in prev.items()}))
+    torch.cuda.synchronize()
+    assert n > 3300
+    for k in ('px', 'py', 'dx_chaotic', 'dy_chaotic'):
+        assert relerr(host(getattr(out, k)), ref[k]) < 1e-12, k

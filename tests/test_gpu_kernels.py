@@ -648,3 +648,107 @@ def test_energy_flux_matches_oracle(precision):
     assert psi.dtype == torch.float64 and psi.is_cuda
     assert ref != 0.0
     assert abs(got - ref) <= 1e-12 * abs(ref)
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
+def test_step_absorbs_in_each_of_its_pushes(precision, monkeypatch):
+    """A plasma step in which the wall absorbs some particles in the first
+    push, others in the second and others in the third, into arrays that held
+    NaN: the first two pushes store the momenta of the absorbed ones only, and
+    every entry is written.  Against the oracle in float64, to the bound of a
+    few tens of steps (ultra-relativistic particles amplify the rounding);
+    in FP32-bulk, where a particle near the threshold may go the other way,
+    every entry is finite and every absorbed particle at rest at its place."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.initialization import init_plasma
+    from lcodepy_amd.plasma3d.solver import Plane2d3vPlasmaSolver
+    N, xi_step = 65, 0.5
+    print(f'step with absorption N={N} {precision}', flush=True)
+    f32 = precision == 'fp32-bulk'
+    rng = np.random.default_rng(78)
+    p = _params(N, xi_step=xi_step)
+    prev, _ = _wall_plasma(rng, p)
+    fields = _edge_quiet_fields(rng, N, p.h)
+    if f32:
+        prev = _round_bulk(prev)
+    _, _, cur_o, const_o, _ = O.init_plasma(p)
+    rb_full, rb_prev = _gauss_beam(N, p.h, -1.0, amp=-10.0), np.zeros((N, N))
+    trace = {}
+    full_o, _, _ = O.step_dxi(p, {'electrons': prev}, fields, cur_o, const_o, rb_full, rb_prev,
+                              trace=trace)
+    full_o = full_o['electrons']
+    gone = [a['q'] == 0 for a in (prev, trace['push1']['electrons'], trace['push2']['electrons'],
+                                  full_o)]
+    new = [int((b & ~a).sum()) for a, b in zip(gone, gone[1:])]
+    print('  absorbed in the pushes:', new, flush=True)
+    assert min(new) > 0
+
+    cfg = _cfg(N, xi_step=xi_step, precision=precision)
+    _, _, cur_g, const_g, _ = init_plasma(cfg)
+    solver = Plane2d3vPlasmaSolver(cfg)
+    parts = {'electrons': _sort_arrays(prev, torch.float32 if f32 else torch.float64)}
+    monkeypatch.setattr(torch, 'empty_like', lambda t: torch.full_like(t, float('nan')))
+    full, _, _ = solver.step_dxi(parts, Arrays.wrap(**{k: dev(v) for k, v in fields.items()}),
+                                 cur_g, const_g, dev(rb_full), dev(rb_prev))
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    solver.ctx.raise_on_errors()
+    full = full['electrons']
+    q = host(full.q)
+    assert not f32 or np.sum((q == 0) != gone[3]) < 0.2 * sum(new)
+    assert f32 or np.array_equal(q == 0, gone[3])
+    for k in ('x_offt', 'y_offt', 'px', 'py', 'pz'):
+        v = host(getattr(full, k))
+        assert np.all(np.isfinite(v)), k
+        assert not np.any(v[q == 0]), k
+        if not f32:
+            assert relerr(v, full_o[k]) < 1e-9, k
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp32-bulk'])
+def test_deposit_of_more_dense_cells_than_a_pass_takes(precision):
+    """More dense cells than the workgroups take at once, lists for a wave and
+    lists for four waves or a workgroup in random turns, so that a workgroup
+    goes from one kind to the other and back; an odd number of the long ones
+    (two are a workgroup's at a time).  Bounds as of the cells at the edges of
+    their lists; two deposits agree bit for bit."""
+    from lcodepy_amd.plasma3d.data import Arrays
+    from lcodepy_amd.plasma3d.weights import get_deposit_plasma
+    print(f'many dense cells {precision}', flush=True)
+    f32 = precision == 'fp32-bulk'
+    N, fineness = 129, 8
+    rng = np.random.default_rng(129)
+    p = _params(N, fineness=fineness)
+    count = np.zeros(N * N, dtype=int)
+    inner = np.arange(N * N).reshape(N, N)[8:N - 8, 8:N - 8].ravel()
+    some = rng.choice(inner, 1101 + 2201, replace=False)
+    count[some[:1101]] = rng.choice([65, 130, 256, 257, 400, 600], 1101)
+    count[some[1101:]] = rng.choice([17, 40, 64], 2201)
+    cell = rng.permutation(np.repeat(np.arange(N * N), count))
+    n = cell.size
+    at = lambda k: (k - N // 2 + 0.98 * rng.uniform(-0.5, 0.5, n)) * p.h
+    m = np.full(n, 0.01)
+    a = dict(x_init=at(cell // N), y_init=at(cell % N), x_offt=np.zeros(n), y_offt=np.zeros(n),
+             q=-m, m=m, **{k: m * rng.normal(0, 0.1, n) for k in ('px', 'py', 'pz')})
+    if f32:
+        a = _round_bulk(a)
+    g = [np.zeros((N, N)) for _ in range(4)]
+    O.deposit_sort(p, a, *g)
+    deposit = get_deposit_plasma(_cfg(N, precision=precision, fineness=fineness))
+    const = Arrays.wrap()
+    const.sorts = {'electrons': 0}
+    parts = {'electrons': _sort_arrays(a, torch.float32 if f32 else torch.float64)}
+    out, again = deposit(parts, const), deposit(parts, const)
+    torch.cuda.synchronize()
+    for u, v, w in zip(out, again, g):
+        assert torch.equal(u, v)
+        assert relerr(host(u[0]), w) < (3e-5 if f32 else 1e-12)
+
+
+@pytest.mark.parametrize('N,precision', [(17, 'fp32-bulk'), (193, 'fp64'), (193, 'fp32-bulk'),
+                                         (257, 'fp64'), (289, 'fp64'), (337, 'fp64'),
+                                         (417, 'fp32-bulk'), (513, 'fp32-bulk')])
+def test_default_launch_shapes_of_the_lds_fft(N, precision):
+    """The FFT solve by default plan and launch shape at lengths 2(N-1) of each
+    of its branches."""
+    test_compute_fields_matches_oracle(N, precision, 'rfft')
