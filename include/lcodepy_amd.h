@@ -98,8 +98,9 @@ typedef struct lc3d_params {
     int32_t field_solver;        /* LC3D_SOLVER_MATRIX, LC3D_SOLVER_FFT or LC3D_SOLVER_RFFT */
     /* LC3D_SOLVER_RFFT launch shape: LDS of a block in complex values, two
      * buffers of half of it (float32 solve: 2048, 4096 or 8192; float64:
-     * 1024, 2048 or 4096; 0 = the largest) and transforms per block, each
-     * taking 2(N-1) values of a buffer (0 = as many as fit) */
+     * 1024, 2048 or 4096) and transforms per block, each taking 2(N-1)
+     * values of a buffer.  Both 0 = library default; one of them 0 = the
+     * largest size, as many as fit */
     int32_t rfft_cap;
     int32_t rfft_tpb;
     /* declustering noise filter of the electrons (plasma3d/noise_filter.py:

@@ -135,26 +135,38 @@ uint64_t rfft_default_plan(int L)
 }
 
 // Default launch shape of the Stockham kernels: complex values of LDS and
-// transforms per block.  Few transforms a block, so that all of the chip's
-// CUs have blocks (7 (N + 1) / 2 transforms a kernel) and a CU holds several;
-// but two where a radix-16 stage of one (L / 16 butterflies) would leave most
-// of the 256 threads idle and the blocks still outnumber the CUs.  Short
-// transforms take the larger LDS size: the smaller one's kernels are compiled
-// for more waves a SIMD and spill.  Measured (default plan, us per solve,
-// this shape against filling the largest LDS size): float32 N = 129 29 (68),
-// 257 39 (76), 417 72 (97), 513 78 (101), 1025 278 (388); float64 129 32 (50),
-// 257 48 (59), 385 94 (101), 513 133, 1025 496.  Float64 transforms of 513 to 682
-// points fill the largest LDS size with three (N = 337 74 us; one a block 82).
-void rfft_default_shape(int L, bool f32, int &cap, int &tpb)
+// transforms per block.  The fewest transforms a block with which all blocks
+// of a kernel (7 fields, ceil(N / 2) transforms each) are resident at once: a
+// block's stages are a chain of waits, so a second round costs nearly the
+// first one's time, and so does a block with twice the transforms.  The
+// smaller LDS size where it holds them (more blocks a CU), but not for a power
+// of two from 256 on, whose radix-16 stages are slower in the fewer registers
+// that its kernels are compiled to (L = 256 33 against 29 us a solve in
+// float32, 36 against 31 in float64).  Where no shape is resident at once: one
+// transform a block, and as many as fit of a power of two.
+// Measured, us per solve, on both sides of the lines (49 sizes were, 33 to 1025,
+// and this rule's shape was the fastest or within 7 % at each).  Float64: N =
+// 209 (735 blocks of one are resident, 768 could be) 49 against 47 with two, 225
+// (791) 53 against 43; 289 (511 of two, 512) 54 against 63 with three, 301 (532)
+// 79 against 69; 351 83 against 95 with two; 513 126 against 119 with two.
+// Float32: 433 (1519 of one, 1536) 64 against 67 with two, 449 (1575) 70 against
+// 65; 513 84 against 72.  Filling the largest LDS size instead: float32 N = 129
+// 61 (29), 257 69 (39), 417 86 (68), 513 89 (72), 1025 333 (250); float64 129
+// 46 (32), 257 55 (46), 385 92 (88).
+void rfft_default_shape(int N, bool f32, int &cap, int &tpb)
 {
-    if (f32) {
-        cap = L > 512 && L < 1024 ? 2048 : 4096;
-        tpb = L == 1024 ? 2 : 1;
-    } else {
-        constexpr int three = 4096 / 6;   // the longest of which three fit a block
-        cap = (L > 256 && L < 512) || (L > three && L < 1024) ? 2048 : 4096;
-        tpb = L == 512 || L == 1024 ? 2 : L > 512 && L <= three ? 4096 / (2 * L) : 1;
+    constexpr int CUS = 256, CAPS[2] = {2048, 4096};
+    const int per_cu[2] = {f32 ? 6 : 3, f32 ? 5 : 2};   // blocks, by registers and by LDS
+    const int L = 2 * (N - 1), pairs = (N + 1) / 2;
+    const bool pow2 = L >= 256 && (L & (L - 1)) == 0;
+    for (tpb = 1; 2 * tpb * L <= CAPS[1]; ++tpb) {
+        for (int c = pow2 ? 1 : 0; c < 2; ++c) {
+            cap = CAPS[c];
+            if (2 * tpb * L <= cap && 7 * ((pairs + tpb - 1) / tpb) <= CUS * per_cu[c]) return;
+        }
     }
+    cap = pow2 || 2 * L > CAPS[0] ? CAPS[1] : CAPS[0];
+    tpb = pow2 ? cap / (2 * L) : 1;
 }
 
 // Packs a caller's plan for the length-L FFT; 0 when it is not one.
@@ -487,7 +499,7 @@ int lc3d_create(const lc3d_params *p, lc3d_ctx **out)
             c->rf_stages = p->fft_nstages > 0 ? rfft_pack_plan(L, p->fft_nstages, p->fft_radix)
                                               : rfft_default_plan(L);
             if (p->rfft_cap <= 0 && p->rfft_tpb <= 0) {
-                rfft_default_shape(L, f32s, c->rf_cap, c->rf_tpb);
+                rfft_default_shape(N, f32s, c->rf_cap, c->rf_tpb);
             } else {
                 c->rf_cap = p->rfft_cap > 0 ? p->rfft_cap : (f32s ? 8192 : 4096);
                 c->rf_tpb = p->rfft_tpb > 0 ? p->rfft_tpb : c->rf_cap / (2 * L);

@@ -746,8 +746,10 @@ def test_deposit_of_more_dense_cells_than_a_pass_takes(precision):
 
 
 @pytest.mark.parametrize('N,precision', [(17, 'fp32-bulk'), (193, 'fp64'), (193, 'fp32-bulk'),
-                                         (257, 'fp64'), (289, 'fp64'), (337, 'fp64'),
-                                         (417, 'fp32-bulk'), (513, 'fp32-bulk')])
+                                         (209, 'fp64'), (225, 'fp64'), (257, 'fp64'),
+                                         (289, 'fp64'), (301, 'fp64'), (337, 'fp64'),
+                                         (351, 'fp64'), (417, 'fp32-bulk'), (433, 'fp32-bulk'),
+                                         (449, 'fp32-bulk'), (513, 'fp32-bulk')])
 def test_default_launch_shapes_of_the_lds_fft(N, precision):
     """The FFT solve by default plan and launch shape at lengths 2(N-1) of each
     of its branches."""
