@@ -95,6 +95,11 @@ class BeamRows(ctypes.Structure):
                 ('i_stride', ctypes.c_int64)]
 
 
+def beam_advance_scratch(n: int) -> int:
+    """Bytes of scratch lc3d_beam_advance needs (LC3D_BEAM_ADVANCE_SCRATCH)."""
+    return 89 * n + 12 * ((n + 31) // 32)
+
+
 class Sort(ctypes.Structure):
     _fields_ = [('n', ctypes.c_int64),
                 ('x_init', _vp), ('y_init', _vp), ('m', _vp),

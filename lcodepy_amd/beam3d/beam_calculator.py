@@ -2,7 +2,7 @@
 from __future__ import annotations
 
 from .. import runtime
-from .._native import BeamRows, ptr, stream_ptr
+from .._native import BeamRows, beam_advance_scratch, ptr, stream_ptr
 from ..config import Config
 from ..plasma3d import _bind
 from .data import FLOAT_KEYS, INT_KEYS, BeamParticles, empty_rounded
@@ -119,7 +119,7 @@ class BeamCalculator:
         for f in (fields_after_layer, fields_before_layer):
             if f.Ex.dtype.itemsize != 8:
                 raise TypeError('the beam moves in the float64 fields of layers k and k+1')
-        scratch_bytes = 89 * n + 12 * ((n + 31) // 32)    # LC3D_BEAM_ADVANCE_SCRATCH
+        scratch_bytes = beam_advance_scratch(n)
         scratch = empty_rounded((scratch_bytes,), torch.uint8, dev)
         out_f = empty_rounded((3, 9, n), torch.float64, dev)
         out_i = empty_rounded((3, 2, n), torch.int64, dev)

@@ -455,15 +455,17 @@ __global__ __launch_bounds__(DENSE_BLOCK) void k_dense_cells(double h, BinState 
 // A grid of fewer blocks of TX = 8, G = 1 than GATHER_FEW takes TX = 4, G = 2:
 // a CU holds several blocks, and each has more waves for its chain.  The
 // second weights cost less than that until the vector units are full.
-// Measured against TX = 8, G = 1 (N = 513: 1235 such blocks, 54.8 us against
-// 56.5 in float64 and 37.2 against 34.3 in float32; 769, 2716, float64, 237
-// against 271; 1025, 4773, float32, 118 against 125) and against TX = 4, G = 1
+// Measured, TX = 8, G = 1 against TX = 4, G = 2 (N = 513, 1368 blocks of the
+// first: 54.8 us against 56.5 in float64 and 37.2 against 34.3 in float32; 769,
+// 2912, float64, 237 against 271; 1025, 5032, float32, 118 against 125), and
+// TX = 4, G = 2 against TX = 4, G = 1
 // (281, 4 ppc, float32, 20.1 us against 26.0; 321 float64 32.4 against 35.0;
 // 129 float64 9.4 against 11.6).
 template <typename T> constexpr int GATHER_FEW = sizeof(T) == 4 ? 2048 : 1024;
 constexpr int GATHER_TY = 28, GATHER_COLS = GATHER_TY + 4;
 static_assert(GATHER_COLS == 32, "a source row is half a wave");
-// cap: records staged at a time (31 KB: five blocks a CU).
+// cap: records staged at a time (31 KB; a block's LDS is 36 to 41 KB in all,
+// four blocks a CU).
 template <typename T> struct GatherPlan {
     static constexpr int cap = sizeof(T) == 4 ? 1280 : 640;
     static_assert(cap >= GATHER_COLS * SMALL_CELL, "one source row always fits");

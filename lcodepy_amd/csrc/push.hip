@@ -57,14 +57,16 @@ __device__ __forceinline__ bool reflect(double x_init, double y_init, double b, 
 // of a few hundred grid points, which the block reads once, coalesced, into
 // LDS, as three pairs of fields (one 16- or 8-byte LDS read gives two
 // fields).  Measured at N = 513, 4 ppc (929,296 particles) inside the step:
-// 76 -> 50 us in float64 and 43 -> 35 us in float32 (the first push 56 ->
-// 38 us, which also no longer needs a pass that rounds the float64 fields),
-// 168 and 124 MB a push, 3.4 and 3.5 TB/s; outside it, in lattice tiles, 80 ->
-// 47 us for 1.1e6 float64 particles.
+// 76 -> 48-50 us in float64 and 43 -> 34-36 us in float32 (the first push 56 ->
+// 35 us, which also no longer needs a pass that rounds the float64 fields), for
+// 207 and 158 MB of HBM traffic a push (counters), 4.2 and 4.5 TB/s; outside it,
+// in lattice tiles, 80 -> 47 us for 1.1e6 float64 particles.
 // A block whose stencils span more than PUSH_WINDOW points (the turn of a
 // strip, a nearly empty region) reads its taps from memory instead.
-// PUSH_WINDOW points take 38 KB in float64: four blocks a CU, as many as the
-// registers allow.
+// PUSH_WINDOW points take 38 KB in float64, 19 in float32: four and five blocks
+// a CU, for which the compiler is held to 128 and 96 registers and spills some
+// of them in the forms that a step runs (float64 28 bytes a lane in the first
+// push and 12 in the others; float32 36 and 12).
 // A sort of fewer than PUSH_FEW particles (STAGED false) leaves CUs idle at
 // PUSH_THREADS a block: there the time is the chain of one wave, which the
 // window only lengthens, so blocks of one wave read their taps from memory.

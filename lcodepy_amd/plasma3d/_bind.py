@@ -23,12 +23,7 @@ def checked_pointers(a, dt) -> list:
 
 
 def check_sort(a, dt) -> None:
-    for k in PARTICLE_KEYS:
-        t = getattr(a, k)
-        want = dt.position if k in POSITION_KEYS else dt.pz if k == 'pz' else dt.bulk
-        if t.dtype != want or not t.is_cuda or not t.is_contiguous():
-            raise TypeError(f'particle array {k}: need a contiguous {want} device tensor, '
-                            f'got {t.dtype} on {t.device}')
+    checked_pointers(a, dt)
 
 
 def sort_struct(prev, full, column: int) -> _native.Sort:

@@ -102,3 +102,24 @@ def test_gpu_library_refuses_the_fft_solver_before_touching_the_device():
     assert not h.value
     p.field_solver = 7
     assert L.lc3d_create(ctypes.byref(p), ctypes.byref(h)) == 1
+
+
+@pytest.mark.skipif(shutil.which('gcc') is None, reason='needs gcc')
+def test_beam_advance_rows_and_scratch_match_the_c_header(tmp_path):
+    sizes = (1, 31, 32, 33, 1000, 2 ** 30)
+    c = tmp_path / 'advance.c'
+    fields = [f for f, _ in _native.BeamRows._fields_]
+    c.write_text('#include <stdio.h>\n#include <stddef.h>\n#include "lcodepy_amd.h"\nint main(void) {\n'
+                 + ''.join(f'printf("%lld\\n", (long long)LC3D_BEAM_ADVANCE_SCRATCH({n}));\n'
+                           for n in sizes)
+                 + ''.join(f'printf("%zu\\n", offsetof(lc3d_beam_rows, {f}));\n' for f in fields)
+                 + 'printf("%zu\\n", sizeof(lc3d_beam_rows)); return 0; }\n')
+    exe = tmp_path / 'advance'
+    subprocess.run(['gcc', '-std=c11', '-I', os.path.dirname(HEADER), str(c), '-o', str(exe)],
+                   check=True)
+    got = [int(v) for v in subprocess.run([str(exe)], capture_output=True, text=True,
+                                          check=True).stdout.split()]
+    want = ([_native.beam_advance_scratch(n) for n in sizes]
+            + [getattr(_native.BeamRows, f).offset for f in fields]
+            + [ctypes.sizeof(_native.BeamRows)])
+    assert got == want
