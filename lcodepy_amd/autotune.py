@@ -1,6 +1,6 @@
 """Field-solve implementation and launch shape chosen by measurement.
 
-``field-solver = 'auto'`` (the default) makes :func:`runtime.context` ask
+``field-solver = 'auto'`` makes :func:`runtime.context` ask
 :func:`solve_choice` which solve to build: ``lc3d_autotune_solve`` times one
 ``compute_fields`` of the run's geometry and precision for the transform-matrix
 products and for the paired LDS FFT over its radix plans, LDS sizes and

@@ -68,8 +68,9 @@ DEFAULT_CONFIG_VALUES: dict[str, Any] = {
     #                  gamma - pz, 1/(1 - v_z) and predictor-corrector averages.
     'precision': 'fp64',
     # Field-solve implementation of the HIP path: 'matrix' (DST-I/DCT-I as
-    # products with N x N transform matrices) or 'fft' (LDS FFTs; only in
-    # libraries built with it, not the GPU library).
+    # products with N x N transform matrices), 'rfft' (paired LDS FFTs), 'auto'
+    # (the faster of these as measured on this GPU) or 'fft' (other LDS FFTs;
+    # only in libraries built with them, not the GPU library).
     'field-solver': 'matrix',
 }
 
@@ -197,10 +198,11 @@ class Config:
                 f"use one of {HIP_PU_TYPES} (this package implements the HIP path only)")
 
     def field_solver(self) -> str:
-        """'auto' (the default: the faster of the two GPU solves for this grid
-        and precision, measured once per process by lcodepy_amd.autotune),
-        'rfft' (paired LDS FFTs), 'matrix' (transform-matrix products on the
-        matrix cores) or 'fft' (refused by the GPU library)."""
+        """'matrix' (transform-matrix products on the matrix cores; the
+        default configuration's), 'rfft' (paired LDS FFTs), 'auto' (the faster
+        of the two for this grid and precision, measured once per process by
+        lcodepy_amd.autotune; taken where a configuration without the defaults
+        has no such key) or 'fft' (refused by the GPU library)."""
         s = self.get('field-solver', 'auto').lower()
         if s not in ('auto', 'matrix', 'fft', 'rfft'):
             raise ValueError(f"field-solver must be 'auto', 'matrix', 'fft' or 'rfft', got {s!r}")
