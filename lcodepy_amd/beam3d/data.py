@@ -8,6 +8,8 @@ Each quantity is a contiguous row view (``beam.x`` ...).  The on-disk /
 exchange record is the reference's ``particle_dtype3d`` (beam3d/data.py:5-7)."""
 from __future__ import annotations
 
+from functools import cached_property
+
 import numpy as np
 
 from ..beam_generator import particle_dtype3d
@@ -51,7 +53,7 @@ class BeamParticles:
             i = torch.zeros(len(INT_KEYS), 0, dtype=torch.int64, device=dev)
         self.f, self.i = f, i
 
-    @property
+    @cached_property
     def xp(self):
         import torch
         return torch

@@ -94,3 +94,16 @@ def test_advance_refuses_rows_it_would_read_past(monkeypatch, part, float_rows, 
     layer, fell = (wrong, none) if part == 'layer' else (none, wrong)
     with pytest.raises(error):
         calc.advance_layer_async(layer, fell, 4, fields, fields)
+
+
+def test_array_module_of_a_beam_can_be_set():
+    """``xp`` is torch until something else is put there, as a class of a
+    caller's may (beam3d/data.py:21-40)."""
+    class Own(BeamParticles):
+        def __init__(self, xp):
+            super().__init__(f=torch.zeros(9, 2), i=torch.zeros(2, 2, dtype=torch.int64))
+            self.xp = xp
+
+    assert BeamParticles(f=torch.zeros(9, 1), i=torch.zeros(2, 1)).xp is torch
+    marker = object()
+    assert Own(marker).xp is marker
